@@ -1009,97 +1009,79 @@ void warm_rain(gwm_state* S, const gwm_warm_rain_config& c, int metric) {
   gwm::launch_warm_rain<R>(S->ctx->stream, a, S->grid->terrain_nonzero);
 }
 
-// Where a reduction keeps its block partials: by default the context's
-// scratch (grown on demand) and a host vector; a caller may pass both.
-struct ReduceBufs {
-  double* dev = nullptr;   // nb * kReduceParts doubles, or null: context scratch
-  double* host = nullptr;  // the same count, or null: a host vector
-};
-
-constexpr int kReduceBlocks = 512;
-static_assert(kReduceBlocks * gwm::kReduceParts <= gwm::kNoAllocScratchDoubles,
-              "the budget partials must fit the static scratch");
-
-// Compensated reduction of one field; returns {sum, min, max, non-finite
-// count} (sum and extremes over the finite values).
+// The budget sums: one launch over every field, then the block records joined
+// on the host in a fixed order.  dev / host: where the records go (both set:
+// the allocation-free form with the static scratch; else the context's
+// scratch and a host vector).
 template <class R>
-void reduce_field(gwm_state* S, const R* f, int fx, int fy, int fz, int kind, const R* rho,
-                  double out[4], const R* fbase = nullptr, const R* rbase = nullptr,
-                  const ReduceBufs& rb = ReduceBufs{}, int halo = -1) {
-  const int nb = kReduceBlocks;
-  const int np = gwm::kReduceParts;
-  double* part = rb.dev ? rb.dev : S->ctx->scratch(static_cast<size_t>(nb) * np);
-  gwm::ReduceArgs<R> a{};
-  a.f = f;
-  a.rho = rho;
-  a.fbase = fbase;
-  a.rbase = rbase;
-  a.cb = S->base<R>();
-  a.idz3 = S->grid->terrain_nonzero ? static_cast<const R*>(S->grid->idz_c) : nullptr;
-  a.idz_lev = static_cast<const R*>(S->grid->lev_idz_c);
-  a.fx = fx;
-  a.fy = fy;
-  a.fz = fz;
-  a.h = halo >= 0 ? halo : S->g().h;
-  a.kind = kind;
-  a.partials = part;
-  if (rb.dev) {
-    gwm::launch_reduce<R>(S->ctx->stream, a, nb);
-    HIPCHK(hipGetLastError());
-  } else {
-    Timed t(S->ctx, "reduce");
-    gwm::launch_reduce<R>(S->ctx->stream, a, nb);
-  }
-  std::vector<double> hv;
-  double* h = rb.host;
-  if (!h) {
-    hv.resize(static_cast<size_t>(nb) * np);
-    h = hv.data();
-  }
-  HIPCHK(hipMemcpyAsync(h, part, static_cast<size_t>(nb) * np * sizeof(double),
-                        hipMemcpyDeviceToHost, S->ctx->stream));
-  HIPCHK(hipStreamSynchronize(S->ctx->stream));
-  double sum = 0.0, comp = 0.0, mn = 1e300, mx = -1e300, bad = 0.0;
-  for (int b = 0; b < nb; ++b) {  // Neumaier over block partials, fixed order
-    for (int q = 0; q < 2; ++q) {
-      const double v = h[b * np + q];
-      const double s2 = sum + v;
-      comp += std::fabs(sum) >= std::fabs(v) ? (sum - s2) + v : (v - s2) + sum;
-      sum = s2;
-    }
-    mn = std::min(mn, h[b * np + 2]);
-    mx = std::max(mx, h[b * np + 3]);
-    bad += h[b * np + 4];
-  }
-  out[0] = sum + comp;
-  out[1] = mn;
-  out[2] = mx;
-  out[3] = bad;
-}
-
-// rb.dev set: the allocation-free form (static scratch, no host vectors;
-// the precipitation bucket is reduced on the device too).
-template <class R>
-void budget(gwm_state* S, double* o, const ReduceBufs& rb = ReduceBufs{}) {
+void budget(gwm_state* S, double* o, double* dev = nullptr, double* host = nullptr) {
   const Geo& g = S->g();
   for (int a = 0; a < GWM_SUMMARY_N; ++a) o[a] = 0.0;
   void** ds = S->cur_set();
-  const R* rho = static_cast<const R*>(ds[0]);
-  const gwm::Base<R> B = S->base<R>();
-  double r[4];
-  // Non-finite values over every prognostic field (the extremes and sums
-  // above are over the finite values only): a field with any NaN or
-  // infinity reports NaN extremes, so no check of them passes by accident.
-  double nonfinite = 0.0;
-  auto extremes = [&](int lo, int hi) {
-    nonfinite += r[3];
-    if (r[3] > 0.0) {
-      o[lo] = std::numeric_limits<double>::quiet_NaN();
-      o[hi] = std::numeric_limits<double>::quiet_NaN();
-    } else {
-      o[lo] = r[1];
-      o[hi] = r[2];
+  gwm::BudgetArgs<R> A{};
+  A.g = g;
+  A.rho = static_cast<const R*>(ds[0]);
+  A.rt = static_cast<const R*>(ds[1]);
+  for (int f = 0; f < 3; ++f) A.face[f] = static_cast<const R*>(ds[GWM_MOM_U + f]);
+  A.ntr = std::min(S->ntr, 3);
+  // (a missing tracer reads rho in its place; its record is not written)
+  for (int t = 0; t < 3; ++t)
+    A.q[t] = t < A.ntr ? static_cast<const R*>(S->field(GWM_TRACER0 + t)) : A.rho;
+  A.precip = static_cast<const R*>(S->view ? S->owner->precip : S->precip);
+  A.idz3 = S->grid->terrain_nonzero ? static_cast<const R*>(S->grid->idz_c) : nullptr;
+  A.idz_lev = static_cast<const R*>(S->grid->lev_idz_c);
+  A.base = S->base<R>();
+  gwm::budget_layout(A);
+  const size_t n = static_cast<size_t>(A.part0[gwm::kBudgetJobs]);
+  require(n <= static_cast<size_t>(gwm::kNoAllocScratchDoubles), "internal: budget records");
+  std::vector<double> hv;
+  if (!host) {
+    hv.resize(n);
+    host = hv.data();
+  }
+  A.part = dev ? dev : S->ctx->scratch(gwm::kNoAllocScratchDoubles);
+  if (dev) {
+    gwm::launch_budget<R>(S->ctx->stream, A);
+    HIPCHK(hipGetLastError());
+  } else {
+    Timed t(S->ctx, "reduce");
+    gwm::launch_budget<R>(S->ctx->stream, A);
+  }
+  scopy(S->ctx->stream, host, A.part, n * sizeof(double), hipMemcpyDeviceToHost);
+
+  // {sum, min, max, non-finite count} of the record at offset q of a job's
+  // blocks: Neumaier over the block sums and compensations, fixed order.
+  struct Rec {
+    double sum, mn, mx, bad;
+  };
+  auto join = [&](int job, int q) -> Rec {
+    double sum = 0.0, comp = 0.0;
+    Rec r{0.0, 1e300, -1e300, 0.0};
+    for (int b = 0; b < A.block0[job + 1] - A.block0[job]; ++b) {
+      const double* h = host + A.part0[job] + static_cast<size_t>(b) * A.record[job] + q;
+      for (int e = 0; e < 2; ++e) {
+        const double s2 = sum + h[e];
+        comp += std::fabs(sum) >= std::fabs(h[e]) ? (sum - s2) + h[e] : (h[e] - s2) + sum;
+        sum = s2;
+      }
+      r.mn = std::min(r.mn, h[2]);
+      r.mx = std::max(r.mx, h[3]);
+      r.bad += h[4];
     }
+    r.sum = sum + comp;
+    return r;
+  };
+  auto count = [&](int job, int q) {
+    double c = 0.0;
+    for (int b = 0; b < A.block0[job + 1] - A.block0[job]; ++b)
+      c += host[A.part0[job] + static_cast<size_t>(b) * A.record[job] + q];
+    return c;
+  };
+  // The extremes and sums are over the finite values: a field with any NaN or
+  // infinity reports NaN extremes, so no check of them passes by accident.
+  auto extremes = [&](int lo, int hi, double mn, double mx, double bad) {
+    o[lo] = bad > 0.0 ? std::numeric_limits<double>::quiet_NaN() : mn;
+    o[hi] = bad > 0.0 ? std::numeric_limits<double>::quiet_NaN() : mx;
   };
   // Perturbation form: sums of the departures plus the FP64 base sums, so
   // the mass budget keeps the departures' precision.
@@ -1118,81 +1100,36 @@ void budget(gwm_state* S, double* o, const ReduceBufs& rb = ReduceBufs{}) {
       base_rt += static_cast<double>(g.nx) * g.ny * bo->base_rt64[static_cast<size_t>(k)];
     }
   }
-  reduce_field<R>(S, rho, g.nx, g.ny, g.nz, 0, nullptr, r, B.rho, nullptr, rb);
-  o[GWM_S_TOTAL_DRY_MASS] = r[0] + base_rho;
-  extremes(GWM_S_RHO_MIN, GWM_S_RHO_MAX);
-  reduce_field<R>(S, static_cast<const R*>(ds[1]), g.nx, g.ny, g.nz, 0, nullptr, r, B.rt,
-                  nullptr, rb);
-  o[GWM_S_TOTAL_RHO_THETA] = r[0] + base_rt;
-  nonfinite += r[3];
-  reduce_field<R>(S, static_cast<const R*>(ds[1]), g.nx, g.ny, g.nz, 2, rho, r, B.rt, B.rho,
-                  rb);
-  const double rt_bad = nonfinite;
-  extremes(GWM_S_THETA_MIN, GWM_S_THETA_MAX);
-  nonfinite = rt_bad;  // theta's non-finite cells are rho's and rho*theta's
-  reduce_field<R>(S, static_cast<const R*>(ds[2]), g.nx + 1, g.ny, g.nz, 0, nullptr, r, nullptr,
-                  nullptr, rb);
-  o[GWM_S_TOTAL_MOM_X] = r[0];
-  extremes(GWM_S_U_MIN, GWM_S_U_MAX);
-  reduce_field<R>(S, static_cast<const R*>(ds[3]), g.nx, g.ny + 1, g.nz, 0, nullptr, r, nullptr,
-                  nullptr, rb);
-  o[GWM_S_TOTAL_MOM_Y] = r[0];
-  extremes(GWM_S_V_MIN, GWM_S_V_MAX);
-  reduce_field<R>(S, static_cast<const R*>(ds[4]), g.nx, g.ny, g.nz + 1, 0, nullptr, r, nullptr,
-                  nullptr, rb);
-  o[GWM_S_TOTAL_MOM_Z] = r[0];
-  extremes(GWM_S_W_MIN, GWM_S_W_MAX);
-  for (int t = 0; t < std::min(S->ntr, 3); ++t) {
-    const R* q = static_cast<const R*>(S->field(GWM_TRACER0 + t));
-    reduce_field<R>(S, q, g.nx, g.ny, g.nz, 1, nullptr, r, nullptr, nullptr, rb);
-    o[GWM_S_VAPOR_PATH + t] = r[0];
-    nonfinite += r[3];
-    const double q_bad = nonfinite;
-    reduce_field<R>(S, q, g.nx, g.ny, g.nz, 2, rho, r, nullptr, B.rho, rb);
-    extremes(GWM_S_TRACER_QMIN0 + 2 * t, GWM_S_TRACER_QMIN0 + 2 * t + 1);
-    nonfinite = q_bad;
+  // Non-finite values over every prognostic field (theta's and the mixing
+  // ratios' non-finite cells are those of the fields they are formed from).
+  double nonfinite = 0.0;
+  const Rec rho = join(0, 0), rt = join(0, 5), th = join(0, 10);
+  o[GWM_S_TOTAL_DRY_MASS] = rho.sum + base_rho;
+  o[GWM_S_TOTAL_RHO_THETA] = rt.sum + base_rt;
+  extremes(GWM_S_RHO_MIN, GWM_S_RHO_MAX, rho.mn, rho.mx, rho.bad);
+  extremes(GWM_S_THETA_MIN, GWM_S_THETA_MAX, th.mn, th.mx, th.bad);
+  nonfinite += rho.bad + rt.bad;
+  for (int f = 0; f < 3; ++f) {
+    const Rec m = join(1 + f, 0);
+    o[GWM_S_TOTAL_MOM_X + f] = m.sum;
+    extremes(GWM_S_U_MIN + 2 * f, GWM_S_U_MAX + 2 * f, m.mn, m.mx, m.bad);
+    nonfinite += m.bad;
   }
-  const size_t n2 = static_cast<size_t>(g.nx) * g.ny;
-  const R* bucket = static_cast<const R*>(S->view ? S->owner->precip : S->precip);
-  if (rb.dev) {
-    // the bucket (ny, nx, no halo) reduced on the device: sum and maximum,
-    // then the count of precipitating columns
-    reduce_field<R>(S, bucket, g.nx, g.ny, 1, 0, nullptr, r, nullptr, nullptr, rb, 0);
-    const double psum = r[0], pmax = r[2];
-    nonfinite += r[3];
-    reduce_field<R>(S, bucket, g.nx, g.ny, 1, 3, nullptr, r, nullptr, nullptr, rb, 0);
-    o[GWM_S_PRECIP_SUM] = psum;
-    o[GWM_S_PRECIP_MEAN] = n2 ? psum / static_cast<double>(n2) : 0.0;
-    o[GWM_S_PRECIP_MAX] = std::max(0.0, pmax);
-    o[GWM_S_PRECIP_CELLS] = static_cast<double>(n2);
-    o[GWM_S_PRECIPITATING_CELLS] = r[0];
-    o[GWM_S_NONFINITE] = nonfinite;
-    return;
+  for (int t = 0; t < A.ntr; ++t) {
+    const Rec q = join(4, 6 * t);
+    o[GWM_S_VAPOR_PATH + t] = q.sum;
+    extremes(GWM_S_TRACER_QMIN0 + 2 * t, GWM_S_TRACER_QMIN0 + 2 * t + 1, q.mn, q.mx,
+             count(4, 6 * t + 5));
+    nonfinite += q.bad;
   }
-  std::vector<R> p(n2);
-  HIPCHK(hipMemcpyAsync(p.data(), bucket, n2 * sizeof(R),
-                        hipMemcpyDeviceToHost, S->ctx->stream));
-  HIPCHK(hipStreamSynchronize(S->ctx->stream));
-  double ps = 0.0, pc = 0.0, pm = 0.0;
-  long wet = 0;
-  for (size_t a = 0; a < n2; ++a) {
-    const double v = static_cast<double>(p[a]);
-    if (!std::isfinite(v)) {
-      nonfinite += 1.0;
-      continue;
-    }
-    const double s2 = ps + v;
-    pc += std::fabs(ps) >= std::fabs(v) ? (ps - s2) + v : (v - s2) + ps;
-    ps = s2;
-    pm = std::max(pm, v);
-    if (v > 0.0) ++wet;
-  }
-  o[GWM_S_PRECIP_SUM] = ps + pc;
-  o[GWM_S_PRECIP_MEAN] = n2 ? (ps + pc) / static_cast<double>(n2) : 0.0;
-  o[GWM_S_PRECIP_MAX] = pm;
-  o[GWM_S_PRECIP_CELLS] = static_cast<double>(n2);
-  o[GWM_S_PRECIPITATING_CELLS] = static_cast<double>(wet);
-  o[GWM_S_NONFINITE] = nonfinite;
+  const Rec p = join(5, 0);
+  const double n2 = static_cast<double>(g.nx) * g.ny;
+  o[GWM_S_PRECIP_SUM] = p.sum;
+  o[GWM_S_PRECIP_MEAN] = p.sum / n2;
+  o[GWM_S_PRECIP_MAX] = std::max(0.0, p.mx);
+  o[GWM_S_PRECIP_CELLS] = n2;
+  o[GWM_S_PRECIPITATING_CELLS] = count(5, 5);
+  o[GWM_S_NONFINITE] = nonfinite + p.bad;
 }
 
 // ---------------------------------------------------------------------------
@@ -2892,11 +2829,8 @@ int gwm_budget_sums_noalloc(gwm_state* s, double* out) {
     require(s->ctx->noalloc, "the context has no budget scratch");
     // host staging on the stack: no allocation on either side
     double host[gwm::kNoAllocScratchDoubles];
-    ReduceBufs rb;
-    rb.dev = s->ctx->noalloc;
-    rb.host = host;
     dispatch(s->ctx, [&](auto r) {
-      budget<decltype(r)>(s, out, rb);
+      budget<decltype(r)>(s, out, s->ctx->noalloc, host);
       return 0;
     });
   });

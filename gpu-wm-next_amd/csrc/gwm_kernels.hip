@@ -511,117 +511,6 @@ __global__ void k_boundary(Geo g, int orient, R* f, const R* ref, int mode, R wi
 }
 
 // ===========================================================================
-// Budget reductions: compensated (Neumaier) FP64 partial sums, min and max
-// of a field over owned elements, optionally weighted by dz = 1/inv_dz_cell
-// (column paths, runtime_summary.cpp:70-80) or divided by rho (mixing
-// ratio, runtime_summary.cpp:82-99).  One partial record per block:
-// {sum, comp, min, max}.
-// ===========================================================================
-template <class R>
-__global__ __launch_bounds__(256) void k_reduce(ReduceArgs<R> a) {
-  __shared__ double sh[256];
-  const int t = threadIdx.x;
-  const size_t n = static_cast<size_t>(a.fx) * a.fy * a.fz;
-  double sum = 0.0, comp = 0.0, mn = 1e300, mx = -1e300, bad = 0.0;
-  for (size_t e = static_cast<size_t>(blockIdx.x) * 256 + t; e < n;
-       e += static_cast<size_t>(gridDim.x) * 256) {
-    const int i = static_cast<int>(e % a.fx);
-    const int j = static_cast<int>((e / a.fx) % a.fy);
-    const int k = static_cast<int>(e / (static_cast<size_t>(a.fx) * a.fy));
-    const size_t idx = (static_cast<size_t>(k) * (a.fy + 2 * a.h) + (j + a.h)) * (a.fx + 2 * a.h) + (i + a.h);
-    double v = static_cast<double>(a.f[idx]);
-    // perturbation form: extremes of the full value, sums of the departure
-    double fb = 0.0;
-    if (a.fbase) {
-      if (a.cb.drho && a.fbase == a.cb.rt)
-        fb = (static_cast<double>(a.cb.rho[k]) + static_cast<double>(a.cb.drho[idx])) *
-             (static_cast<double>(a.cb.th[k]) + static_cast<double>(a.cb.dth[idx]));
-      else
-        fb = static_cast<double>(a.fbase[k]) + (a.cb.drho ? static_cast<double>(a.cb.drho[idx]) : 0.0);
-    }
-    const double full = a.fbase ? v + fb : v;
-    double ext = full;
-    if (a.kind == 1) {  // column path
-      const R idz = a.idz3 ? a.idz3[(static_cast<size_t>(k) * a.fy + j) * a.fx + i] : a.idz_lev[k];
-      v = v * (1.0 / static_cast<double>(idz));
-      ext = v;
-    } else if (a.kind == 2) {  // theta_m / mixing ratio: f / max(rho, 1e-12)
-      const double r = static_cast<double>(a.rho[idx]) +
-                       (a.rbase ? static_cast<double>(a.rbase[k]) +
-                                      (a.cb.drho ? static_cast<double>(a.cb.drho[idx]) : 0.0)
-                                : 0.0);
-      v = full / fmax(r, 1.0e-12);
-      ext = v;
-    } else if (a.kind == 3) {  // count of positive values; extremes of the value
-      v = full > 0.0 ? 1.0 : 0.0;
-    }
-    // A NaN or infinity is counted, and kept out of the sums and extremes,
-    // which then describe the finite values; the count tells the caller
-    // whether those describe the whole field.
-    if (!isfinite(full) || !isfinite(v)) {
-      bad += 1.0;
-      continue;
-    }
-    const double s2 = sum + v;
-    comp += fabs(sum) >= fabs(v) ? (sum - s2) + v : (v - s2) + sum;
-    sum = s2;
-    mn = fmin(mn, ext);
-    mx = fmax(mx, ext);
-  }
-  // Block combine in a fixed tree order; every node is a TwoSum whose
-  // rounding error joins the compensation, so sum + comp stays exact to
-  // working precision.
-  double* out = a.partials + static_cast<size_t>(blockIdx.x) * kReduceParts;
-  __shared__ double se[256];
-  sh[t] = sum;
-  se[t] = comp;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) {
-      const double x = sh[t], y = sh[t + s];
-      const double s2 = x + y;
-      const double bb = s2 - x;
-      const double err = (x - (s2 - bb)) + (y - bb);
-      sh[t] = s2;
-      se[t] = se[t] + se[t + s] + err;
-    }
-    __syncthreads();
-  }
-  const double bsum = sh[0];
-  const double bcomp = se[0];
-  __syncthreads();
-  sh[t] = mn;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) sh[t] = fmin(sh[t], sh[t + s]);
-    __syncthreads();
-  }
-  const double bmn = sh[0];
-  __syncthreads();
-  sh[t] = mx;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) sh[t] = fmax(sh[t], sh[t + s]);
-    __syncthreads();
-  }
-  const double bmx = sh[0];
-  __syncthreads();
-  sh[t] = bad;  // counts below 2^53 add exactly in any order
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) sh[t] += sh[t + s];
-    __syncthreads();
-  }
-  if (t == 0) {
-    out[0] = bsum;
-    out[1] = bcomp;
-    out[2] = bmn;
-    out[3] = bmx;
-    out[4] = sh[0];
-  }
-}
-
-// ===========================================================================
 // Metric construction (grid_metrics.hpp:184-236): one thread per column,
 // FP64 arithmetic without contraction so the stored values match a host
 // build of the same formulas.
@@ -809,12 +698,6 @@ void launch_boundary(hipStream_t st, const Geo& g, int orient, R* f, const R* re
   hipLaunchKernelGGL(k_boundary<R>, dim3(blocks_for(n, 256)), dim3(256), 0, st, g, orient, f, ref,
                      mode, static_cast<R>(width), wx, wy);
 }
-template <class R>
-void launch_reduce(hipStream_t st, const ReduceArgs<R>& a, int nblocks) {
-  if (refuse_record("reduce")) return;
-  hipLaunchKernelGGL(k_reduce<R>, dim3(nblocks), dim3(256), 0, st, a);
-}
-
 Recorder*& recorder() {
   static thread_local Recorder* r = nullptr;
   return r;
@@ -876,7 +759,6 @@ void launch_fill(hipStream_t st, R* dst, size_t n, R v) {
   template void launch_sync_interfaces<R>(hipStream_t, const Geo&, int, R*);                     \
   template void launch_exchange_layout<R>(hipStream_t, int, int, int, const int*, R* const*, int); \
   template void launch_boundary<R>(hipStream_t, const Geo&, int, R*, const R*, int, double);     \
-  template void launch_reduce<R>(hipStream_t, const ReduceArgs<R>&, int);                        \
   template void launch_metrics<R>(hipStream_t, const Geo&, const double*, const double*,         \
                                   const double*, const double*, const float*, R*, R*, R*, R*, R*, \
                                   R*, R*);                                                        \

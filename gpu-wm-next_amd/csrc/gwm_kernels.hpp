@@ -75,26 +75,30 @@ struct WarmRainArgs {
   Base<R> base;  // perturbation form
 };
 
-// Per-block partials of k_reduce: sum, compensation, min, max and the count
-// of non-finite values.
-constexpr int kReduceParts = 5;
-
+// Budget sums (gwm_budget.hip).  Jobs: cells (rho, rho*theta), the three face
+// fields, tracers, the bucket; work-groups block0[job] .. block0[job+1) write
+// one record of record[job] doubles each, at part + part0[job]:
+//   cells    rho, rho*theta, theta: {sum, compensation, min, max, non-finite} each
+//   faces    the same five
+//   tracers  {path sum, compensation, ratio min, max, path non-finite, ratio non-finite} each
+//   bucket   the five, then the count of positive columns
+constexpr int kBudgetJobs = 6;
 template <class R>
-struct ReduceArgs {
-  const R* f;
-  const R* rho;
-  const R* idz3;
-  const R* idz_lev;
-  int fx, fy, fz, h;
-  int kind;  // 0 value, 1 value*dz, 2 value/rho, 3 count of values > 0
-  double* partials;
-  // Perturbation form: per-level bases added for min / max (and for rho in
-  // kind 2); sums stay over the stored departures.  On terrain (cb.drho set)
-  // the cell's base is the level value plus its deviation; rho*theta's is
-  // rho_b theta_b of the cell's.
-  const R* fbase;
-  const R* rbase;
-  Base<R> cb;
+struct BudgetArgs {
+  Geo g;
+  const R *rho, *rt;
+  const R* face[3];
+  const R* q[3];
+  int ntr;  // tracers summed (at most 3)
+  const R* precip;
+  const R* idz3;     // 1 / dz per cell on terrain, else null
+  const R* idz_lev;  // 1 / dz per level
+  // Perturbation form: sums are over the stored departures, extremes of the
+  // full values (on terrain the cell's base is the level value plus its
+  // deviation; rho*theta's is rho_b theta_b of the cell's).
+  Base<R> base;
+  double* part;
+  int block0[kBudgetJobs + 1], part0[kBudgetJobs + 1], record[kBudgetJobs];
 };
 
 template <class R>
@@ -146,8 +150,12 @@ void launch_exchange_layout(hipStream_t st, int phase, int orient, int nranks, c
 template <class R>
 void launch_boundary(hipStream_t st, const Geo& g, int orient, R* f, const R* ref, int mode,
                      double width);
+// Divides the work-groups among the jobs; returns their number.  The records
+// take part0[kBudgetJobs] doubles, at most kNoAllocScratchDoubles.
 template <class R>
-void launch_reduce(hipStream_t st, const ReduceArgs<R>& a, int nblocks);
+int budget_layout(BudgetArgs<R>& a);
+template <class R>
+void launch_budget(hipStream_t st, const BudgetArgs<R>& a);
 
 // Plan-view products (gwm-next-plan-view/v1, src/io/plan_view_output.cpp),
 // in the reference's field order: 10 dry fields, 3 with specific humidity,
@@ -181,7 +189,7 @@ struct PlanViewArgs {
 template <class R>
 void launch_plan_view(hipStream_t st, const PlanViewArgs<R>& a, bool terrain);
 
-// Allocation-free budget sums: k_reduce block partials live in a static
+// Allocation-free budget sums: the block records live in a static
 // device array of kNoAllocScratchDoubles doubles (32 KiB), one per GPU.
 constexpr int kNoAllocScratchDoubles = 4096;
 constexpr int kNoAllocMaxDevices = 64;

@@ -379,7 +379,7 @@ int gwm_plan_view(gwm_state* state, int slice_k, int steps, double dt, int with_
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  The reduction partials live
  * in a static device array of 4096 doubles (32 KiB per GPU, held until the
- * process ends; the budget needs 512 x 5 of them for any grid size), host
+ * process ends; the budget needs fewer of them for any grid size), host
  * staging is on the stack, and the precipitation bucket is reduced on the
  * device.  Same slots as gwm_budget_sums: counts, extremes and the
  * non-finite count agree exactly, sums to rounding (the bucket is summed in
