@@ -2925,7 +2925,7 @@ int gwm_init_convection(gwm_state* s, double p_s, unsigned long long seed, doubl
 struct gwm_surrogate {
   gwm_ctx* ctx = nullptr;
   gwm::SurTrain T;
-  int batch = 0;  // rows the training buffers hold
+  int grad_groups = 0;  // work-groups whose gradient partials T.gpart holds
   gwm::SurNorm norm{};
   bool have_norm = false;
   long version = 0;  // bumped by set_norm (graphs bake the normalisation in)
@@ -2936,39 +2936,22 @@ struct gwm_surrogate {
   size_t loss_n = 0;
   ~gwm_surrogate() {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
-    free_batch();
     for (void* p : {static_cast<void*>(T.params), static_cast<void*>(T.grad),
-                    static_cast<void*>(T.m), static_cast<void*>(T.v),
+                    static_cast<void*>(T.m), static_cast<void*>(T.v), static_cast<void*>(T.gpart),
                     static_cast<void*>(nfall), static_cast<void*>(loss_part)})
       if (p) (void)hipFree(p);
     ctx_release(ctx);
   }
-  void free_batch() {
-    std::vector<float*> ps = {T.xn, T.wpart};
-    for (auto* q : T.z) ps.push_back(q);
-    for (auto* q : T.a) ps.push_back(q);
-    for (auto* q : T.dz) ps.push_back(q);
-    for (float* q : ps)
-      if (q) (void)hipFree(q);
-    T.xn = T.wpart = nullptr;
-    for (auto& q : T.z) q = nullptr;
-    for (auto& q : T.a) q = nullptr;
-    for (auto& q : T.dz) q = nullptr;
-    batch = 0;
-  }
+  // Gradient partials for minibatches of up to B rows.
   void ensure_batch(int B) {
-    if (B <= batch) return;
-    free_batch();
-    auto fa = [](size_t n) { return static_cast<float*>(dalloc(n * sizeof(float))); };
-    T.xn = fa(static_cast<size_t>(B) * 8);
-    for (int l = 0; l < 4; ++l) {
-      const size_t w = l < 3 ? 64 : gwm::kSurOut;
-      T.z[l] = fa(static_cast<size_t>(B) * w);
-      T.dz[l] = fa(static_cast<size_t>(B) * w);
-      if (l < 3) T.a[l] = fa(static_cast<size_t>(B) * 64);
-    }
-    T.wpart = fa(static_cast<size_t>(16) * 65 * 64);
-    batch = B;
+    const int groups = gwm::sur_grad_groups(B);
+    if (groups <= grad_groups) return;
+    if (T.gpart) HIPCHK(hipFree(T.gpart));
+    T.gpart = nullptr;
+    grad_groups = 0;
+    T.gpart = static_cast<float*>(
+        dalloc(static_cast<size_t>(groups) * gwm::kSurParams * sizeof(float)));
+    grad_groups = groups;
   }
   double* loss_buf(size_t n) {
     if (n > loss_n) {
@@ -3184,7 +3167,7 @@ int gwm_surrogate_train(gwm_surrogate* m, const void* dev_x, const void* dev_y, 
     require(lr > 0.0 && lr_final > 0.0, "learning rates must be positive");
     m->ensure_batch(batch);
     const long nmb = n / batch;
-    const int per = (batch * gwm::kSurOut + 255) / 256;
+    const int per = gwm::sur_grad_groups(batch);
     double* part = m->loss_buf(static_cast<size_t>(nmb) * per);
     const long total = nmb * epochs;
     const float* X = static_cast<const float*>(dev_x);
@@ -3196,10 +3179,9 @@ int gwm_surrogate_train(gwm_surrogate* m, const void* dev_x, const void* dev_y, 
         // cosine decay from lr to lr_final over all steps
         const double f = 0.5 * (1.0 + std::cos(M_PI * static_cast<double>(step) / total));
         m->T.lr = static_cast<float>(lr_final + (lr - lr_final) * f);
-        int nl = 0;
         gwm::launch_sur_train_step(m->ctx->stream, m->T, X + b * batch * gwm::kSurIn,
                                    Y + b * batch * gwm::kSurOut, batch, m->norm, true,
-                                   part + b * per, &nl);
+                                   part + b * per);
       }
       HIPCHK(hipGetLastError());
       HIPCHK(hipMemcpyAsync(h.data(), part, h.size() * sizeof(double), hipMemcpyDeviceToHost,
@@ -3219,11 +3201,10 @@ int gwm_surrogate_loss_grad(gwm_surrogate* m, const void* dev_x, const void* dev
     require(m->have_norm, "surrogate normalisation not set");
     require(n >= 1, "need at least one row");
     m->ensure_batch(n);
-    const int per = (n * gwm::kSurOut + 255) / 256;
-    double* part = m->loss_buf(static_cast<size_t>(per));
-    int nl = 0;
+    const int nl = gwm::sur_grad_groups(n);
+    double* part = m->loss_buf(static_cast<size_t>(nl));
     gwm::launch_sur_train_step(m->ctx->stream, m->T, static_cast<const float*>(dev_x),
-                               static_cast<const float*>(dev_y), n, m->norm, false, part, &nl);
+                               static_cast<const float*>(dev_y), n, m->norm, false, part);
     HIPCHK(hipGetLastError());
     std::vector<double> h(static_cast<size_t>(nl));
     HIPCHK(hipMemcpyAsync(h.data(), part, h.size() * sizeof(double), hipMemcpyDeviceToHost,

@@ -23,19 +23,10 @@ namespace {
 constexpr float kGeluA = 0.7978845608028654f;  // sqrt(2 / pi)
 constexpr float kGeluB = 0.044715f;
 
-__device__ inline float gelu_f(float x) {
-  const float u = kGeluA * (x + kGeluB * x * x * x);
-  return 0.5f * x * (1.0f + tanhf(u));
-}
-__device__ inline float gelu_grad_f(float x) {
-  const float u = kGeluA * (x + kGeluB * x * x * x);
-  const float t = tanhf(u);
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * kGeluA * (1.0f + 3.0f * kGeluB * x * x);
-}
-// Same function as gelu_f written as x * sigmoid(2u) = x / (1 + 2^(x (c0 +
-// c1 x^2))), c0 = -2 A log2(e), c1 = c0 B, for inference: seven instructions
-// (hardware exp2 and reciprocal), within a few FP32 ulp of gelu_f, far below
-// the BF16 rounding that follows.
+// GELU (tanh form, u = A (x + B x^3)) written as x * sigmoid(2u) = x / (1 +
+// 2^(x (c0 + c1 x^2))), c0 = -2 A log2(e), c1 = c0 B, for inference: seven
+// instructions (hardware exp2 and reciprocal), within a few FP32 ulp of
+// x/2 (1 + tanh u), far below the BF16 rounding that follows.
 __device__ inline float gelu_fast(float x) {
   constexpr float c0 = -2.0f * kGeluA * 1.44269504088896341f;
   constexpr float c1 = c0 * kGeluB;
@@ -99,102 +90,233 @@ __global__ void k_sur_sample(Geo g, const float* rho, const float* rt, const flo
 }
 
 // ===========================================================================
-// FP32 training kernels.  Row-major activations [B][width].
+// FP32 training: one launch computes a minibatch's loss and gradient, a
+// second sums the gradient over its work-groups and applies Adam.
+//
+// A work-group of four waves takes tiles of 32 rows through the forward pass
+// and back with v_mfma_f32_16x16x4_f32 (FP32 operands and accumulation): wave
+// w owns the 16 neurons 16 w .. 16 w + 15 of every hidden layer, so its
+// slices of the weights and of their transposes stay in registers, and only
+// activations and layer gradients pass through LDS (rows of 68 floats: a
+// thread's 16 values of a row are four aligned 16-byte reads).  The k order of
+// a product is free as long as both operands share it: step s of lane group g
+// stands for k = 16 g + s (rows 8 g + s in the weight gradients).  The weight
+// gradients accumulate in registers over a work-group's tiles.
+//
+// A step is about 215 MFLOP for 4096 rows, two microseconds of FP32 matrix
+// rate: it is bound by the chain of layers and the launches.  As eighteen
+// launches of one thread per output (weight gradients as 256-row serial sums)
+// an epoch of 65536 rows in batches of 4096 took 6.97 ms; it takes 0.44 ms.
 // ===========================================================================
+namespace {
 
-// x_n[b][0..7] = (x[b][f] - mean) / std, feature 7 = 0.
-__global__ void k_sur_norm_in(const float* x, long n, SurNorm nm, float* xn) {
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= n * 8) return;
-  const long b = t >> 3;
-  const int f = static_cast<int>(t & 7);
-  xn[t] = f < kSurIn ? (x[b * kSurIn + f] - nm.xm[f]) / nm.xs[f] : 0.0f;
+typedef float f32v4 __attribute__((ext_vector_type(4)));
+
+constexpr int kRows = 32;      // rows of a tile
+constexpr int kPitch = 64 + 4; // LDS row pitch in floats
+constexpr int kGradGroups = 256;  // most work-groups of a gradient launch
+
+__device__ inline f32v4 mfma4(float a, float b, f32v4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// z = in W + b; a = gelu(z) (act) or z.  Thread per (row, out).
-__global__ void k_dense_fwd(const float* in, int ldi, int K, const float* W, const float* bias,
-                            int N, int B, int act, float* z, float* a) {
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<long>(B) * N) return;
-  const long b = t / N;
-  const int n = static_cast<int>(t % N);
-  float s = bias[n];
-  const float* row = in + b * ldi;
-  for (int k = 0; k < K; ++k) s += row[k] * W[k * N + n];
-  z[t] = s;
-  if (a) a[t] = act ? gelu_f(s) : s;
-}
-
-// dy = 2 (y_pred - y_target_n) / (B * 4); per-block partial loss sums.
-__global__ __launch_bounds__(256) void k_mse_grad(const float* yp, const float* yt, int B,
-                                                  SurNorm nm, float* dy, double* part) {
-  __shared__ double sh[256];
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  double l = 0.0;
-  if (t < static_cast<long>(B) * kSurOut) {
-    const int o = static_cast<int>(t % kSurOut);
-    const float target = (yt[t] - nm.ym[o]) / nm.ys[o];
-    const float d = yp[t] - target;
-    dy[t] = 2.0f * d / static_cast<float>(B * kSurOut);
-    l = static_cast<double>(d) * d;
+// acc += rows [row0, row0 + 16) of a staged [kRows][64] array times the wave's
+// 64 x 16 weight slice (w[s]: k = 16 g + s).
+__device__ inline f32v4 dense64(const float (*in)[kPitch], int row0, const float (&w)[16], int c,
+                                int g, f32v4 acc) {
+  const f32v4* r = reinterpret_cast<const f32v4*>(&in[row0 + c][16 * g]);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32v4 v = r[q];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma4(v[e], w[4 * q + e], acc);
   }
-  sh[threadIdx.x] = l;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+  return acc;
+}
+
+}  // namespace
+
+// Loss (sum of squared normalised errors per work-group) and gradient partials
+// gpart[work-group][kSurParams] of rows [0, B).
+__global__ __launch_bounds__(256) void k_sur_grad(const float* p, const float* x, const float* y,
+                                                  int B, SurNorm nm, float* gpart,
+                                                  double* loss_part) {
+  __shared__ float sx[kRows][8], d4[kRows][4];
+  __shared__ __align__(16) float a1[kRows][kPitch], a2[kRows][kPitch], a3[kRows][kPitch];
+  __shared__ __align__(16) float d1[kRows][kPitch], d2[kRows][kPitch], d3[kRows][kPitch];
+  __shared__ double sl[2];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int c = lane & 15, g = lane >> 4, n = 16 * w + c;
+  // the wave's weight slices: forward (k, n), backward transposed (n, k)
+  float w1[2], w2[16], w3[16], w4[16], t2[16], t3[16];
+  for (int s = 0; s < 2; ++s) w1[s] = 2 * g + s < kSurIn ? p[kSurW1 + (2 * g + s) * 64 + n] : 0.0f;
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    const int k = 16 * g + s;
+    w2[s] = p[kSurW2 + k * 64 + n];
+    w3[s] = p[kSurW3 + k * 64 + n];
+    t2[s] = p[kSurW2 + n * 64 + k];
+    t3[s] = p[kSurW3 + n * 64 + k];
+    w4[s] = c < kSurOut ? p[kSurW4 + k * kSurOut + c] : 0.0f;
+  }
+  const float t4 = p[kSurW4 + n * kSurOut + g];
+  const float b1 = p[kSurB1 + n], b2 = p[kSurB2 + n], b3 = p[kSurB3 + n];
+  const float b4 = c < kSurOut ? p[kSurB4 + c] : 0.0f;
+  const f32v4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32v4 gw1 = zero, gw2[4], gw3[4], gw4 = zero, gb1 = zero, gb2 = zero, gb3 = zero, gb4 = zero;
+  for (int q = 0; q < 4; ++q) gw2[q] = gw3[q] = zero;
+  double loss = 0.0;
+
+  // activation and its derivative of the wave's 16 x 16 output tile
+  auto act = [&](const f32v4& z, int row0, float (*a)[kPitch], f32v4& dg) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float v = z[r], u = kGeluA * (v + kGeluB * v * v * v), th = tanhf(u);
+      a[row0 + 4 * g + r][n] = 0.5f * v * (1.0f + th);
+      dg[r] = 0.5f * (1.0f + th) +
+              0.5f * v * (1.0f - th * th) * kGeluA * (1.0f + 3.0f * kGeluB * v * v);
+    }
+  };
+  // weight gradient of a 64 x 64 layer: inputs in (rows x k), gradients d
+  auto grad64 = [&](const float (*in)[kPitch], const float (*d)[kPitch], f32v4 (&gw)[4], f32v4& gb) {
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int row = 8 * g + s;
+      const float dv = d[row][n];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) gw[q] = mfma4(in[row][16 * q + c], dv, gw[q]);
+      gb = mfma4(1.0f, dv, gb);
+    }
+  };
+
+  for (int tile = blockIdx.x; tile * kRows < B; tile += gridDim.x) {
+    {
+      const int row = t >> 3, f = t & 7, r = tile * kRows + row;
+      sx[row][f] = f < kSurIn && r < B ? (x[static_cast<size_t>(r) * kSurIn + f] - nm.xm[f]) / nm.xs[f]
+                                       : 0.0f;
+    }
     __syncthreads();
+    f32v4 dg1[2], dg2[2], dg3[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      f32v4 z = {b1, b1, b1, b1};
+      for (int s = 0; s < 2; ++s) z = mfma4(sx[16 * h + c][2 * g + s], w1[s], z);
+      act(z, 16 * h, a1, dg1[h]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      act(dense64(a1, 16 * h, w2, c, g, f32v4{b2, b2, b2, b2}), 16 * h, a2, dg2[h]);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      act(dense64(a2, 16 * h, w3, c, g, f32v4{b3, b3, b3, b3}), 16 * h, a3, dg3[h]);
+    __syncthreads();
+    if (w < 2) {  // outputs of row half w, their error and its gradient
+      const f32v4 z = dense64(a3, 16 * w, w4, c, g, f32v4{b4, b4, b4, b4});
+      if (c < kSurOut) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * w + 4 * g + r, gr = tile * kRows + row;
+          float dz = 0.0f;
+          if (gr < B) {
+            const float d = z[r] - (y[static_cast<size_t>(gr) * kSurOut + c] - nm.ym[c]) / nm.ys[c];
+            dz = 2.0f * d / static_cast<float>(B * kSurOut);
+            loss += static_cast<double>(d) * d;
+          }
+          d4[row][c] = dz;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int row = 8 * g + s;
+      const float dv = c < kSurOut ? d4[row][c] : 0.0f;
+      gw4 = mfma4(a3[row][n], dv, gw4);
+      gb4 = mfma4(1.0f, dv, gb4);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32v4 da = mfma4(d4[16 * h + c][g], t4, zero);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d3[16 * h + 4 * g + r][n] = da[r] * dg3[h][r];
+    }
+    __syncthreads();
+    grad64(a2, d3, gw3, gb3);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32v4 da = dense64(d3, 16 * h, t3, c, g, zero);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d2[16 * h + 4 * g + r][n] = da[r] * dg2[h][r];
+    }
+    __syncthreads();
+    grad64(a1, d2, gw2, gb2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const f32v4 da = dense64(d2, 16 * h, t2, c, g, zero);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d1[16 * h + 4 * g + r][n] = da[r] * dg1[h][r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int row = 8 * g + s;
+      const float dv = d1[row][n];
+      gw1 = mfma4(c < 8 ? sx[row][c] : 0.0f, dv, gw1);
+      gb1 = mfma4(1.0f, dv, gb1);
+    }
+    __syncthreads();  // the next tile replaces the staged features
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+
+  float* out = gpart + static_cast<size_t>(blockIdx.x) * kSurParams;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = 16 * q + 4 * g + r;
+      out[kSurW2 + k * 64 + n] = gw2[q][r];
+      out[kSurW3 + k * 64 + n] = gw3[q][r];
+    }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int k = 4 * g + r;
+    if (k < kSurIn) out[kSurW1 + k * 64 + n] = gw1[r];
+    if (c < kSurOut) out[kSurW4 + (16 * w + k) * kSurOut + c] = gw4[r];
+  }
+  if (g == 0) {
+    out[kSurB1 + n] = gb1[0];
+    out[kSurB2 + n] = gb2[0];
+    out[kSurB3 + n] = gb3[0];
+    if (w == 0 && c < kSurOut) out[kSurB4 + c] = gb4[0];
+  }
+  loss = wave_sum_to63(loss);
+  if (w < 2 && lane == 63) sl[w] = loss;
+  __syncthreads();
+  if (t == 0) loss_part[blockIdx.x] = sl[0] + sl[1];
 }
 
-// dz_in[b][k] = (sum_n dz[b][n] W[k][n]) * gelu'(z_in[b][k]).
-__global__ void k_dense_bwd_data(const float* dz, int N, const float* W, int K, const float* zin,
-                                 int B, float* dzin) {
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<long>(B) * K) return;
-  const long b = t / K;
-  const int k = static_cast<int>(t % K);
+// Gradient = sum of the work-groups' partials, then (update) one Adam step.
+// Eight threads to a parameter, each with its partials' loads in flight
+// together; fixed summation order.
+__global__ __launch_bounds__(512) void k_sur_update(const float* gpart, int groups, float* grad,
+                                                    int update, float* p, float* m, float* v,
+                                                    float lr, float b1, float b2, float eps,
+                                                    float c1, float c2) {
+  __shared__ float sh[8][64];
+  const int q = threadIdx.x & 63, sl = threadIdx.x >> 6;
+  const int t = blockIdx.x * 64 + q;
+  const int tc = t < kSurParams ? t : kSurParams - 1;
   float s = 0.0f;
-  const float* row = dz + b * N;
-  for (int n = 0; n < N; ++n) s += row[n] * W[k * N + n];
-  dzin[t] = s * gelu_grad_f(zin[t]);
-}
-
-// Partial weight gradients over a slice of the batch: out[slice][k][n]
-// (k == K is the bias row).  Fixed summation order.
-__global__ void k_dense_bwd_weight(const float* in, int ldi, int K, const float* dz, int N, int B,
-                                   int slices, float* out) {
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const long per = static_cast<long>(K + 1) * N;
-  if (t >= per * slices) return;
-  const int sl = static_cast<int>(t / per);
-  const int kn = static_cast<int>(t % per);
-  const int k = kn / N, n = kn % N;
-  const int b0 = static_cast<int>((static_cast<long>(B) * sl) / slices);
-  const int b1 = static_cast<int>((static_cast<long>(B) * (sl + 1)) / slices);
-  float s = 0.0f;
-  for (int b = b0; b < b1; ++b) s += (k < K ? in[static_cast<long>(b) * ldi + k] : 1.0f) * dz[static_cast<long>(b) * N + n];
-  out[t] = s;
-}
-
-// g[W offset + k*N + n] / g[b offset + n] = sum over slices.
-__global__ void k_dense_grad_reduce(const float* part, int K, int N, int slices, float* gW,
-                                    float* gb) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int per = (K + 1) * N;
-  if (t >= per) return;
-  float s = 0.0f;
-  for (int sl = 0; sl < slices; ++sl) s += part[static_cast<long>(sl) * per + t];
-  const int k = t / N, n = t % N;
-  if (k < K) gW[k * N + n] = s;
-  else gb[n] = s;
-}
-
-__global__ void k_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1,
-                       float b2, float eps, float c1, float c2) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float gt = g[t];
+#pragma unroll 16
+  for (int k = sl; k < groups; k += 8) s += gpart[static_cast<size_t>(k) * kSurParams + tc];
+  sh[sl][q] = s;
+  __syncthreads();
+  if (sl != 0 || t >= kSurParams) return;
+  const float gt = ((sh[0][q] + sh[1][q]) + (sh[2][q] + sh[3][q])) +
+                   ((sh[4][q] + sh[5][q]) + (sh[6][q] + sh[7][q]));
+  grad[t] = gt;
+  if (!update) return;
   const float mt = b1 * m[t] + (1.0f - b1) * gt;
   const float vt = b2 * v[t] + (1.0f - b2) * gt * gt;
   m[t] = mt;
@@ -716,55 +838,26 @@ void launch_sur_sample(hipStream_t st, const Geo& g, const float* rho, const flo
                      mc, seed, n, x, y, cell, base);
 }
 
+int sur_grad_groups(int B) {
+  const int tiles = (B + kRows - 1) / kRows;
+  return tiles < kGradGroups ? tiles : kGradGroups;
+}
+
 void launch_sur_train_step(hipStream_t st, SurTrain& T, const float* x, const float* y, int B,
-                           const SurNorm& nm, bool update, double* loss_part, int* nloss) {
+                           const SurNorm& nm, bool update, double* loss_part) {
   if (refuse_record("sur_train_step")) return;
-  float* p = T.params;
-  // forward
-  hipLaunchKernelGGL(k_sur_norm_in, dim3(nblk(static_cast<long>(B) * 8, 256)), dim3(256), 0, st,
-                     x, static_cast<long>(B), nm, T.xn);
-  const float* in = T.xn;
-  int ldi = 8, K = kSurIn;
-  const int wofs[4] = {kSurW1, kSurW2, kSurW3, kSurW4};
-  const int bofs[4] = {kSurB1, kSurB2, kSurB3, kSurB4};
-  for (int l = 0; l < 4; ++l) {
-    const int N = l < 3 ? 64 : kSurOut;
-    hipLaunchKernelGGL(k_dense_fwd, dim3(nblk(static_cast<long>(B) * N, 256)), dim3(256), 0, st,
-                       in, ldi, K, p + wofs[l], p + bofs[l], N, B, l < 3 ? 1 : 0, T.z[l],
-                       l < 3 ? T.a[l] : nullptr);
-    in = l < 3 ? T.a[l] : nullptr;
-    ldi = 64;
-    K = 64;
-  }
-  // loss and output gradient
-  const unsigned lb = nblk(static_cast<long>(B) * kSurOut, 256);
-  hipLaunchKernelGGL(k_mse_grad, dim3(lb), dim3(256), 0, st, T.z[3], y, B, nm, T.dz[3],
+  const int groups = sur_grad_groups(B);
+  hipLaunchKernelGGL(k_sur_grad, dim3(groups), dim3(256), 0, st, T.params, x, y, B, nm, T.gpart,
                      loss_part);
-  if (nloss) *nloss = static_cast<int>(lb);
-  // backward
-  const int slices = 16;
-  for (int l = 3; l >= 0; --l) {
-    const int N = l < 3 ? 64 : kSurOut;
-    const int Kl = l == 0 ? kSurIn : 64;
-    const float* inl = l == 0 ? T.xn : T.a[l - 1];
-    const int ldl = l == 0 ? 8 : 64;
-    const long parts = static_cast<long>(Kl + 1) * N * slices;
-    hipLaunchKernelGGL(k_dense_bwd_weight, dim3(nblk(parts, 256)), dim3(256), 0, st, inl, ldl,
-                       Kl, T.dz[l], N, B, slices, T.wpart);
-    hipLaunchKernelGGL(k_dense_grad_reduce, dim3(nblk(static_cast<long>(Kl + 1) * N, 256)),
-                       dim3(256), 0, st, T.wpart, Kl, N, slices, T.grad + wofs[l],
-                       T.grad + bofs[l]);
-    if (l > 0)
-      hipLaunchKernelGGL(k_dense_bwd_data, dim3(nblk(static_cast<long>(B) * 64, 256)), dim3(256),
-                         0, st, T.dz[l], N, p + wofs[l], 64, T.z[l - 1], B, T.dz[l - 1]);
-  }
+  float c1 = 1.0f, c2 = 1.0f;
   if (update) {
     T.step += 1;
-    const float c1 = 1.0f - powf(T.beta1, static_cast<float>(T.step));
-    const float c2 = 1.0f - powf(T.beta2, static_cast<float>(T.step));
-    hipLaunchKernelGGL(k_adam, dim3(nblk(kSurParams, 256)), dim3(256), 0, st, p, T.grad, T.m, T.v,
-                       kSurParams, T.lr, T.beta1, T.beta2, T.eps, c1, c2);
+    c1 = 1.0f - powf(T.beta1, static_cast<float>(T.step));
+    c2 = 1.0f - powf(T.beta2, static_cast<float>(T.step));
   }
+  hipLaunchKernelGGL(k_sur_update, dim3(nblk(kSurParams, 64)), dim3(512), 0, st, T.gpart, groups,
+                     T.grad, update ? 1 : 0, T.params, T.m, T.v, T.lr, T.beta1, T.beta2, T.eps, c1,
+                     c2);
 }
 
 void launch_sur_infer(hipStream_t st, const float* w, const SurNorm& nm, const float* x, long n,

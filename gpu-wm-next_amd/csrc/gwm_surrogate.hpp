@@ -27,17 +27,13 @@ struct SurNorm {
   float lo[kSurIn], hi[kSurIn];
 };
 
-// Device buffers of the FP32 training path for a minibatch of B rows.
+// Device buffers of the FP32 training path.
 struct SurTrain {
   float* params = nullptr;  // kSurParams (master weights)
   float* grad = nullptr;
   float* m = nullptr;
   float* v = nullptr;
-  float* xn = nullptr;  // [B][8]
-  float* z[4] = {};     // pre-activations [B][64] (z[3]: [B][4] outputs)
-  float* a[3] = {};     // activations [B][64]
-  float* dz[4] = {};    // gradients w.r.t. z
-  float* wpart = nullptr;  // [16][65][64] partial weight gradients
+  float* gpart = nullptr;  // [sur_grad_groups(B)][kSurParams] gradient partials
   long step = 0;
   float lr = 1.0e-3f, beta1 = 0.9f, beta2 = 0.999f, eps = 1.0e-8f;
 };
@@ -46,11 +42,13 @@ void launch_sur_sample(hipStream_t st, const Geo& g, const float* rho, const flo
                        const float* qv, const float* qc, const float* qr,
                        const MicroCfg<float>& mc, unsigned long long seed, long n, float* x,
                        float* y, long long* cell, Base<float> base);
+// Work-groups of the gradient launch for B rows.
+int sur_grad_groups(int B);
 // Forward + loss + backward on B rows (x raw [B][7], y raw [B][4]); with
-// `update`, one Adam step.  Per-block loss partials (sum of squared
-// normalised errors) go to loss_part, their count to *nloss.
+// `update`, one Adam step.  sur_grad_groups(B) loss partials (sums of squared
+// normalised errors) go to loss_part.
 void launch_sur_train_step(hipStream_t st, SurTrain& T, const float* x, const float* y, int B,
-                           const SurNorm& nm, bool update, double* loss_part, int* nloss);
+                           const SurNorm& nm, bool update, double* loss_part);
 void launch_sur_infer(hipStream_t st, const float* w, const SurNorm& nm, const float* x, long n,
                       float* y);
 // Arguments of the surrogate warm-rain call.  The call runs in two passes:

@@ -302,3 +302,27 @@ def test_split_fallout_equals_whole_column_fallout(ctx, metric):
     # rain reaches the ground in columns of both kinds
     assert np.all(pb[cols] > 0) and np.any(pb[~cols] > 0)
     assert np.allclose(pa, pb, rtol=1e-6, atol=1e-12 * np.max(pb))
+
+
+@pytest.mark.parametrize("n", [1, 15, 32, 33, 100, 8192 + 17])
+def test_loss_and_gradient_at_tile_edges(ctx, n):
+    """Row counts below, at and past a 32-row tile, and past one tile per
+    work-group (256 of them), against the FP64 oracle (bars as above: FP32
+    sums, the terms' rounding grows with their number, not their order)."""
+    _, st = small_state(ctx, seed=4)
+    X, Y, _ = sample(ctx, st, n, seed=12)
+    x, y = X.download(), Y.download()
+    rows = np.concatenate([x, x * np.float32(1.1)])  # a spread for n = 1
+    norm = _norm_of(rows, np.concatenate([y, y + np.float32(1e-3)]))
+    sur = G.Surrogate(ctx, seed=5)
+    sur.set_norm(**norm)
+    p = SO.init_xavier(9).astype(np.float32)
+    sur.set_params(p)
+    loss, grad = sur.loss_grad(X, Y, n)
+    n32 = {k: np.asarray(v, np.float32).astype(np.float64) for k, v in sur.norm().items()}
+    ref_loss, ref_grad = SO.loss_grad(p.astype(np.float64), x, y, n32, fp32_normalise=True)
+    assert abs(loss - ref_loss) <= 1e-5 * ref_loss, (loss, ref_loss)
+    for lo, hi in ((0, 448), (448, 512), (512, 4608), (4608, 4672), (4672, 8768), (8768, 8832),
+                   (8832, 9088), (9088, 9092)):
+        r = np.linalg.norm(grad[lo:hi] - ref_grad[lo:hi]) / np.linalg.norm(ref_grad[lo:hi])
+        assert r < 1e-4, (lo, r)
