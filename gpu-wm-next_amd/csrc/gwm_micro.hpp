@@ -35,13 +35,17 @@ __device__ inline MicroCell<R> micro_prepare(R rho_raw, R rt0, R rqv, R rqc, R r
   MicroCell<R> m;
   m.rho = rmax(rho_raw, R(1.0e-6));
   m.th = qdiv(rt0, m.rho);
-  m.p = q_pressure(m.rho, rt0);
-  m.T = q_theta(m.rho, rt0) * qpow(rmax(qdiv(m.p, Phys<R>::p0), R(1.0e-6)), Phys<R>::kappa);
-  const R ex = rmax(qdiv(m.T, rmax(m.th, R(1.0e-6))), R(1.0e-6));
+  R exner;
+  m.p = q_pressure_exner(m.rho, rt0, exner);
+  m.T = m.th * exner;
+  // T / max(theta, 1e-6), floored (FP64: the Exner function itself)
+  R ex;
+  if constexpr (sizeof(R) == 8) ex = rmax(exner * rmin(m.th * R(1.0e6), R(1)), R(1.0e-6));
+  else ex = rmax(qdiv(m.T, rmax(m.th, R(1.0e-6))), R(1.0e-6));
   m.qv = rmax(qdiv(rqv, m.rho), R(0));
   m.qc = rmax(qdiv(rqc, m.rho), R(0));
   m.qr = rmax(qdiv(rqr, m.rho), R(0));
-  m.lfac = qdiv(Phys<R>::Lv, d_cp<R>() * rmax(ex, R(1.0e-6)));
+  m.lfac = qdiv(Phys<R>::Lv, d_cp<R>() * ex);
   return m;
 }
 
@@ -73,8 +77,9 @@ __device__ inline void micro_apply(MicroCell<R>& m, const MicroCfg<R>& c) {
     qc -= ac;
     qr += ac;
   }
-  const R p = q_pressure(rho, rho * th);
-  const R T = th * qpow(rmax(qdiv(p, Phys<R>::p0), R(1.0e-6)), Phys<R>::kappa);
+  R exner;
+  const R p = q_pressure_exner(rho, rho * th, exner);
+  const R T = th * exner;
   qs = q_qsat(T, p);
   if (qr > R(0) && qv < qs && c.erate > R(0)) {
     const R e = rmin(qr, c.dt * c.erate * rmin(qs - qv, qr));
