@@ -201,6 +201,7 @@ struct gwm_grid {
       if (p) (void)hipFree(p);
     ctx_release(ctx);
   }
+  size_t metric_total() const { return static_cast<size_t>(geo.nx) * geo.ny * geo.nz; }
   template <class R>
   DMetrics<R> dm() const {
     return DMetrics<R>{static_cast<const R*>(zc_m), static_cast<const R*>(idz_c),
@@ -306,6 +307,7 @@ struct gwm_state {
   void* theta_ref = nullptr;  // nz
   void* rref_lev = nullptr;   // nz
   void* pref_lev = nullptr;   // nz
+  void* ref3 = nullptr;       // column reference (terrain): rho, then p, per cell
   void* theta_scr = nullptr;  // cell field
   // FP64 level partial sums of the step (theta_ref, fast-mode level means):
   // owned by the state and sized once for its grid, so the step graphs
@@ -378,7 +380,7 @@ struct gwm_state {
       b.push_back(reinterpret_cast<const void*>(v->size()));
       for (const void* q : *v) b.push_back(q);
     }
-    for (const void* q : {pressure, precip, theta_ref, rref_lev, pref_lev, theta_scr, b_dev, b3_dev,
+    for (const void* q : {pressure, precip, theta_ref, rref_lev, pref_lev, ref3, theta_scr, b_dev, b3_dev,
                           bf_dev, static_cast<void*>(step_part), static_cast<void*>(sur_queue)})
       b.push_back(q);
     return b;
@@ -459,7 +461,7 @@ struct gwm_state {
     for (auto* v : {&tr, &tr_scr[0], &tr_scr[1], &tr_scr[2], &bref_tr})
       for (void* p : *v)
         if (p) (void)hipFree(p);
-    for (void* p : {pressure, precip, theta_ref, rref_lev, pref_lev, theta_scr, b_dev, b3_dev, bf_dev,
+    for (void* p : {pressure, precip, theta_ref, rref_lev, pref_lev, ref3, theta_scr, b_dev, b3_dev, bf_dev,
                     static_cast<void*>(step_part), static_cast<void*>(sur_queue)})
       if (p) (void)hipFree(p);
   }
@@ -612,6 +614,7 @@ int subcycle(gwm_state* S, const gwm_step_config& c, const R* rho_in, const R* t
     if (!S->rref_lev) S->rref_lev = dalloc(g.nz * sizeof(R));
     if (!S->pref_lev) S->pref_lev = dalloc(g.nz * sizeof(R));
   }
+  if (colref && !S->ref3) S->ref3 = dalloc(2 * G->metric_total() * sizeof(R));
   const int outs[2] = {z0, z1};
   const R* rho = rho_in;
   const R *u = ub, *v = vb, *w = wb;  // departures after the first substep
@@ -650,6 +653,8 @@ int subcycle(gwm_state* S, const gwm_step_config& c, const R* rho_in, const R* t
     a.w_out = static_cast<R*>(S->set[o][4]);
     a.rref_lev = static_cast<const R*>(S->rref_lev);
     a.pref_lev = static_cast<const R*>(S->pref_lev);
+    a.rref3 = static_cast<R*>(S->ref3);
+    a.pref3 = colref ? a.rref3 + G->metric_total() : nullptr;
     a.m = G->dm<R>();
     a.dtf = dtf;
     a.gravity = static_cast<R>(c.gravity);
@@ -673,12 +678,9 @@ int subcycle(gwm_state* S, const gwm_step_config& c, const R* rho_in, const R* t
       gwm::launch_fast_column<R>(S->ctx->stream, a, G->terrain_nonzero, n,
                                  emit ? part : nullptr, emit ? &nparts : nullptr);
     };
-    // flat launches choose level chunks and the tile height (8 or 4 rows);
-    // column-reference launches keep whole columns and choose the height
-    const int nkc =
-        colref ? pick_chunks(S->ctx, "fast_column", g, 2, run, 2, /*whole_columns=*/true)
-               : pick_chunks(S->ctx, "fast_column", g, G->terrain_nonzero ? (tp ? 3 : 1) : 0, run,
-                             G->terrain_nonzero ? 1 : 2);
+    // level chunks and tile height (8 or 4 rows) per form
+    const int nkc = pick_chunks(S->ctx, "fast_column", g,
+                                colref ? 2 : G->terrain_nonzero ? (tp ? 3 : 1) : 0, run, 2);
     Timed t(S->ctx, "fast_column");
     run(nkc);
     rho = a.rho_out;

@@ -36,6 +36,7 @@ struct FastArgs {
   R *rho_out, *u_out, *v_out, *w_out;  // face departures, full faces if last
   R* rt_out;  // rho*theta rebuild (last substep), may be null
   const R *rref_lev, *pref_lev;  // flat reference (nz)
+  R *rref3, *pref3;  // column reference (metric layout; col_ref), scratch of the launch
   DMetrics<R> m;
   R dtf, gravity;
   int horizontal, density, col_ref;
@@ -122,8 +123,8 @@ void launch_slow_column(hipStream_t st, const SlowArgs<R>& a, bool terrain, int 
 // also writes the next substep's level partials, one per 64-column row
 // segment, [k][row][tile column][2], and returns their count per level in
 // *nparts.  code: level chunks per column in the low 4 bits (1 = whole
-// columns; the column-reference path keeps 1) and, in bit 4, a tile height
-// of 4 rows instead of 8 (flat launches without the column reference).
+// columns) and, in bit 4, a tile height of 4 rows instead of 8.  With col_ref
+// the column reference is built first, by a launch of its own.
 template <class R>
 void launch_fast_column(hipStream_t st, const FastArgs<R>& a, bool terrain, int code,
                         double* part_out, int* nparts);
@@ -263,6 +264,11 @@ struct FastItem {
   FastArgs<R> a;
   int tiles_x, tiles, nkc;
   double* part_out;
+  int gx, gy;
+};
+template <class R>
+struct ColumnRefItem {
+  FastArgs<R> a;
   int gx, gy;
 };
 template <class R>
