@@ -227,10 +227,14 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
   };
   // Own-column rho (levels k-1, k, k+1), rho*theta (k, k+1) and the top w face.
   R r_km1 = R(0), r_k = R(0), r_k1 = R(0), rt_k = R(0), rt_k1 = R(0), w_top = R(0);
+  // (terrain perturbation form: the base deviations of the same)
+  R br_km1 = R(0), br_k = R(0), br_k1 = R(0), bt_k = R(0), bt_k1 = R(0);
   auto stage_lev = [&](const Lev& q, int kk) {
     stage_raw(q.o, eo, kk);
     r_k1 = q.o.r;
     rt_k1 = q.o.rt;
+    br_k1 = q.o.br;
+    bt_k1 = q.o.bt;
     if (kk + 1 == nz) w_top = q.o.w1;
     if (t < NHALO) stage_raw(q.h, eh, kk);
   };
@@ -269,16 +273,71 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
     return static_cast<size_t>(L.mj(jj)) * g.nx + L.mi(ii);
   };
 
+  // Terrain metrics of the own column and of the ones west and south of it
+  // (the other columns of the cell's x and y face): heights of levels k-1, k
+  // and k+1 (clamped to the column) are carried, the rest of a level is
+  // loaded a level early (FP32).  Read where they were used, these were 13
+  // loads a level in front of which a wave waited: the perturbation form's
+  // stage of 192 x 192 x 60 took 124 us, and takes 96.  FP64 reads them where
+  // they are used: carrying them costs it 40 more registers, and the stage of
+  // 151 x 97 x 40 went from 72 to 104 us with them.
+  constexpr bool MET = TERRAIN && sizeof(R) == 4;
+  struct Met {
+    R z[3];                // height of level k+1
+    R idz[3], idz_f;       // of the cells, and of the own z face, at level k
+    R fu, fv;              // base forcing of the x and y face at level k
+  };
+  struct Heights {
+    R lo[3], at[3], hi[3];
+  };
+  const unsigned pm = static_cast<unsigned>(g.nx) * g.ny;
+  unsigned mc[3] = {0, 0, 0};
+  if constexpr (MET) {
+    mc[0] = static_cast<unsigned>(mcol(i, j));
+    mc[1] = static_cast<unsigned>(mcol(i - 1, j));
+    mc[2] = static_cast<unsigned>(mcol(i, j - 1));
+  }
+  auto load_met = [&](int kk) -> Met {
+    Met q{};
+    if constexpr (MET) {
+      const unsigned up = static_cast<unsigned>(kk + 1 < nz ? kk + 1 : nz - 1) * pm;
+      const unsigned here = static_cast<unsigned>(kk) * pm;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        q.z[c] = ld32(a.m.zc, mc[c] + up);
+        q.idz[c] = ld32(a.m.idz_c, mc[c] + here);
+      }
+      q.idz_f = ld32(a.m.idz_f, mc[0] + here);
+    }
+    if constexpr (TP) {
+      q.fu = ld32(a.base.fu, q0x + static_cast<unsigned>(kk) * pu);
+      q.fv = ld32(a.base.fv, q0y + static_cast<unsigned>(kk) * pv);
+    }
+    return q;
+  };
+
   // highest level a chunk stages (uniform; kept in a scalar register so the
   // clamped level indices and their offsets stay scalar work)
   const int kcap = __builtin_amdgcn_readfirstlane(k1 < nz - 1 ? k1 : nz - 1);
+  Met MA = load_met(k0);
+  Heights H{};
+  if constexpr (MET) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      H.at[c] = ld32(a.m.zc, mc[c] + static_cast<unsigned>(k0 > 0 ? k0 - 1 : 0) * pm);
+      H.hi[c] = ld32(a.m.zc, mc[c] + static_cast<unsigned>(k0) * pm);
+    }
+  }
   if (k0 > 0) {
     stage_lev(load_lev(k0 - 1), k0 - 1);
     r_km1 = r_k1;
+    br_km1 = br_k1;
   }
   stage_lev(load_lev(k0), k0);
   r_k = r_k1;
   rt_k = rt_k1;
+  br_k = br_k1;
+  bt_k = bt_k1;
   // FP32 pipelines the raw loads a level ahead; FP64 (twice the registers per
   // value) loads each level where it stages it.
   constexpr bool PIPE = sizeof(R) == 4;
@@ -298,15 +357,25 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
   struct Carry {
     R m, th, thb, u, v, w;
   } cz{};
-  auto level = [&](int k, const Lev& Ln, Lev& Lnn) {
+  auto level = [&](int k, const Lev& Ln, Lev& Lnn, const Met& Mc, Met& Mn) {
     Q0 Qc;
     if constexpr (PIPE) {
       if (k + 1 < nz) stage_lev(Ln, k + 1);
       Qc = load_q0(k);
+      Mn = load_met(k + 1 < k1 ? k + 1 : k);
       Lnn = load_lev(k + 2 < kcap ? k + 2 : kcap);
     } else {
       if (k + 1 < nz) stage_lev(load_lev(k + 1), k + 1);
       Qc = load_q0(k);
+      Mn = load_met(k + 1 < k1 ? k + 1 : k);
+    }
+    if constexpr (MET) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        H.lo[c] = H.at[c];
+        H.at[c] = H.hi[c];
+        H.hi[c] = Mc.z[c];
+      }
     }
     __syncthreads();
     if (active) {
@@ -348,10 +417,6 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         if (TERRAIN) return a.m.idz_c[mcol(ii, jj) + kk * plane_m];
         return LV(kk, SL_IDZC);
       };
-      auto IDZF = [&](int ii, int jj, int kk) -> R {
-        if (TERRAIN) return a.m.idz_f[mcol(ii, jj) + kk * plane_m];
-        return LV(kk, SL_IDZF);
-      };
       // dp/dz at column (ii, jj) (dry_pressure_gradient.cu:37-73).
       auto vgrad = [&](int ii, int jj) -> R {
         if (nz == 1) return R(0);
@@ -369,13 +434,26 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         return qdiv(P(ii, jj, k + 1) - P(ii, jj, k - 1), rmax(dz, R(1.0e-6)));
       };
 
+      // The same of the own (0), west (1) and south (2) column, whose heights
+      // are carried: with the clamped levels, one expression at every level.
+      auto grad = [&](int c, int ii, int jj) -> R {
+        if constexpr (!MET) return vgrad(ii, jj);
+        return qdiv(P(ii, jj, kt) - P(ii, jj, kb), rmax(H.hi[c] - H.lo[c], R(1.0e-6)));
+      };
+      auto height = [&](int c, int ii, int jj) -> R {
+        if constexpr (!MET) return a.m.zc[mcol(ii, jj) + k * plane_m];
+        return H.at[c];
+      };
+      auto idz_cell = [&](int c, int ii, int jj) -> R {
+        if constexpr (!MET) return IDZC(ii, jj, k);
+        return Mc.idz[c];
+      };
       // The own column's dp/dz and height enter its x face and its y face
-      // (and the domain-edge faces): evaluated once, the same arithmetic as
-      // at each face.
+      // (and the domain-edge faces): evaluated once.
       R g_own = R(0), z_own = R(0);
       if constexpr (TERRAIN) {
-        g_own = vgrad(i, j);
-        z_own = a.m.zc[mcol(i, j) + k * plane_m];
+        g_own = grad(0, i, j);
+        z_own = height(0, i, j);
       }
 
       // ---- K2 (dry_core.cu:62-144)
@@ -387,7 +465,7 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         // top face's of the level before (carried, bit for bit the same)
         const bool carried = k > k0;
         const R mb = carried ? cz.m : W(i, j, k), mt = w_up;
-        const R idz = IDZC(i, j, k);
+        const R idz = idz_cell(0, i, j);
         const R div = qdivc(me - mw, dx, rdx) + qdivc(mn - ms, dy, rdy) + (mt - mb) * idz;
         t_rho = -div;
         const R thc = TH(i, j, k);
@@ -449,21 +527,29 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         const R ft0 = upwind(R(0.5) * (WC(fi - 1, j, k) + WC(fi, j, k)), qc, qt);
         if (carry) *carry = ft0;
         const R fb = k > 0 ? fb0 : R(0), ft = k + 1 < nz ? ft0 : R(0);
-        const R idz = TERRAIN ? R(0.5) * (IDZC(fi - 1, j, k) + IDZC(fi, j, k)) : IDZC(fi, j, k);
+        const bool own_r = carry != nullptr;  // the face between the west and the own column
+        const R idz = !TERRAIN ? LV(k, SL_IDZC)
+                      : own_r  ? R(0.5) * (idz_cell(1, i - 1, j) + idz_cell(0, i, j))
+                               : R(0.5) * (idz_cell(0, i, j) + IDZC(fi, j, k));
         const R A = -(qdivc(fe - fw, dx, rdx) + qdivc(fn - fs, dy, rdy) + (ft - fb) * idz);
         const R pl = P(fi - 1, j, k), pr = P(fi, j, k);
         R term;
         if (TERRAIN) {
           // face fi lies between columns fi-1 and fi, one of them the own
           // (fi == i: the right one; the edge face nx: the left one)
-          const bool own_r = fi == i;
-          const int nb = own_r ? fi - 1 : fi;
-          const R zn = a.m.zc[mcol(nb, j) + k * plane_m], gn = vgrad(nb, j);
+          R zn, gn;
+          if (own_r) {
+            zn = height(1, i - 1, j);
+            gn = grad(1, i - 1, j);
+          } else {
+            zn = a.m.zc[mcol(fi, j) + k * plane_m];
+            gn = vgrad(fi, j);
+          }
           const R zl = own_r ? zn : z_own, zr = own_r ? z_own : zn;
           const R gl = own_r ? gn : g_own, gr = own_r ? g_own : gn;
           const R dzdx = qdivc(zr - zl, dx, rdx);
           term = qdivc(pr - pl, dx, rdx) - dzdx * (R(0.5) * (gl + gr));
-          if constexpr (TP) term = term + ld32(a.base.fu, fo);
+          if constexpr (TP) term = term + (own_r ? Mc.fu : ld32(a.base.fu, fo));
         } else {
           term = qdivc(pr - pl, dx, rdx);
         }
@@ -490,19 +576,27 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         const R ft0 = upwind(R(0.5) * (WC(i, fj - 1, k) + WC(i, fj, k)), qc, qt);
         if (carry) *carry = ft0;
         const R fb = k > 0 ? fb0 : R(0), ft = k + 1 < nz ? ft0 : R(0);
-        const R idz = TERRAIN ? R(0.5) * (IDZC(i, fj - 1, k) + IDZC(i, fj, k)) : IDZC(i, fj, k);
+        const bool own_n = carry != nullptr;
+        const R idz = !TERRAIN ? LV(k, SL_IDZC)
+                      : own_n  ? R(0.5) * (idz_cell(2, i, j - 1) + idz_cell(0, i, j))
+                               : R(0.5) * (idz_cell(0, i, j) + IDZC(i, fj, k));
         const R A = -(qdivc(fe - fw, dx, rdx) + qdivc(fn - fs, dy, rdy) + (ft - fb) * idz);
         const R ps = P(i, fj - 1, k), pn = P(i, fj, k);
         R term;
         if (TERRAIN) {
-          const bool own_n = fj == j;
-          const int nb = own_n ? fj - 1 : fj;
-          const R zb = a.m.zc[mcol(i, nb) + k * plane_m], gb = vgrad(i, nb);
+          R zb, gb;
+          if (own_n) {
+            zb = height(2, i, j - 1);
+            gb = grad(2, i, j - 1);
+          } else {
+            zb = a.m.zc[mcol(i, fj) + k * plane_m];
+            gb = vgrad(i, fj);
+          }
           const R zs = own_n ? zb : z_own, zn = own_n ? z_own : zb;
           const R gs = own_n ? gb : g_own, gnn = own_n ? g_own : gb;
           const R dzdy = qdivc(zn - zs, dy, rdy);
           term = qdivc(pn - ps, dy, rdy) - dzdy * (R(0.5) * (gs + gnn));
-          if constexpr (TP) term = term + ld32(a.base.fv, fo);
+          if constexpr (TP) term = term + (own_n ? Mc.fv : ld32(a.base.fv, fo));
         } else {
           term = qdivc(pn - ps, dy, rdy);
         }
@@ -532,7 +626,7 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         }
         const R ft = upwind(WC(i, j, ku), qc, qt);
         cz.w = ft;
-        const R idz = IDZF(i, j, k);
+        const R idz = MET ? Mc.idz_f : TERRAIN ? a.m.idz_f[mcol(i, j) + k * plane_m] : LV(k, SL_IDZF);
         const R A = -(qdivc(fe - fw, dx, rdx) + qdivc(fn - fs, dy, rdy) + (ft - fb) * idz);
         const R tf = R(0.5) * (TH(i, j, kl) + TH(i, j, ku));
         if (pert) {
@@ -541,8 +635,8 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
           R rl = r_km1 + LV(kl, SL_BRHO);
           R ru = r_k + LV(ku, SL_BRHO);
           if constexpr (TP) {  // the cell's base: level value + deviation
-            rl = r_km1 + (LV(kl, SL_BRHO) + ld32(a.base.drho, oc0 + static_cast<unsigned>(kl) * pc));
-            ru = r_k + (LV(ku, SL_BRHO) + ld32(a.base.drho, oc0 + static_cast<unsigned>(ku) * pc));
+            rl = r_km1 + (LV(kl, SL_BRHO) + br_km1);
+            ru = r_k + (LV(ku, SL_BRHO) + br_k);
           }
           const R trp = R(0.5) * (LV(kl, SL_TREF) + LV(ku, SL_TREF));
           const R trf = R(0.5) * (LV(kl, SL_BTH) + LV(ku, SL_BTH)) + trp;
@@ -580,8 +674,8 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
         // floors on the full values (departures: 1e-6 - base)
         R rbk = LV(k, SL_BRHO), tbk = LV(k, SL_BTH), rtbk = LV(k, SL_BRT);
         if constexpr (TP) {  // the own cell's base
-          rbk = rbk + ld32(a.base.drho, ci);
-          tbk = tbk + ld32(a.base.dth, ci);
+          rbk = rbk + br_k;
+          tbk = tbk + bt_k;
           rtbk = rbk * tbk;
         }
         const R flr = pert ? R(1.0e-6) - rbk : R(1.0e-6);
@@ -609,11 +703,15 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
     r_km1 = r_k;
     r_k = r_k1;
     rt_k = rt_k1;
+    br_km1 = br_k;
+    br_k = br_k1;
+    bt_k = bt_k1;
   };
   Lev LB{};
+  Met MB{};
   for (int k = k0; k < k1; k += 2) {
-    level(k, LA, LB);
-    if (k + 1 < k1) level(k + 1, LB, LA);
+    level(k, LA, LB, MA, MB);
+    if (k + 1 < k1) level(k + 1, LB, LA, MB, MA);
   }
 }
 
