@@ -254,19 +254,28 @@ __global__ void k_rebuild_rt(Geo g, const R* rho, const R* th, R* rt, Base<R> ba
 }
 
 // ===========================================================================
-// Warm rain + fallout, one thread per column marching top-down: K24
-// (warm_rain.cu:36-120) on cell k, then the fallout sweep on the same cell
-// (K25 nominal, warm_rain.cu:122-154, or K26 metric, 156-191), which reads
-// the post-microphysics rain exactly like the reference's qr_old copy.
+// Warm rain + fallout, marching columns top-down: K24 (warm_rain.cu:36-120)
+// on cell k, then the fallout sweep on the same cell (K25 nominal,
+// warm_rain.cu:122-154, or K26 metric, 156-191), which reads the
+// post-microphysics rain exactly like the reference's qr_old copy.
+//
+// A wave is 64 columns, and the waves of a work-group share them, each with a
+// chunk of the levels (blockDim.y chunks): what falls into a chunk depends on
+// the level above it only, which the wave adjusts a second time for itself.
+// The update is in place, so every wave reads that level before any writes
+// (they are all in the work-group).  One thread per column left too few waves
+// to cover the loads (figures at the launcher's rule).
 // ===========================================================================
 template <class R, bool TERRAIN>
 __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const VBlock& vb) {
   const Geo g = a.g;
   int bx, by;
   xcd_block2d(vb, bx, by);
-  const int i = bx * blockDim.x + threadIdx.x;
-  const int j = by * blockDim.y + threadIdx.y;
-  if (i >= g.nx || j >= g.ny) return;
+  const int ic = bx * 64 + static_cast<int>(threadIdx.x), j = by;
+  const bool in = ic < g.nx;
+  const int i = in ? ic : g.nx - 1;
+  const int nch = static_cast<int>(blockDim.y), chunk = static_cast<int>(threadIdx.y);
+  const int k0 = (g.nz * chunk) / nch, k1 = (g.nz * (chunk + 1)) / nch;
   const R dt = a.dt;
   R inc = 0;
   const R dz_nom = rmax(a.depth, R(1.0e-3));
@@ -276,38 +285,28 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
   const bool nominal = a.fallout == 1 && frac_nom > R(0), metric = a.fallout == 2;
   const R rdz_nom = R(1) / dz_nom;
   const MicroCfg<R> mc{dt, a.relax, a.thr, a.krate, a.erate, a.kacc, a.heat};
-  // The loads of the level three below are issued before the current
-  // level's arithmetic: three levels of loads in flight per column keep
-  // enough requests outstanding at one column per thread.
   const size_t plane = static_cast<size_t>(g.pxc) * g.pyc;
-  size_t c = g.cell(i, j, g.nz - 1);
   struct Lv {
     R rho, rt, qv, qc, qr;
   };
   auto load = [&](size_t cc) -> Lv { return {a.rho[cc], a.rt[cc], a.qv[cc], a.qc[cc], a.qr[cc]}; };
-  Lv l1 = load(c), l2{}, l3{};
-  if (g.nz > 1) l2 = load(c - plane);
-  if (g.nz > 2) l3 = load(c - 2 * plane);
   const bool pert = a.base.rho != nullptr;
-  for (int k = g.nz - 1; k >= 0; --k) {
-    const Lv cur = l1;
-    l1 = l2;
-    l2 = l3;
-    if (k >= 3) l3 = load(c - 3 * plane);
-    // Perturbation form: full rho and rho*theta for the microphysics; the
-    // stored departure of rho*theta then changes by rho * dtheta only.
-    const R rtp = cur.rt;
+  // The adjusted cell: perturbation form: full rho and rho*theta for the
+  // microphysics; the stored departure of rho*theta then changes by rho *
+  // dtheta only.
+  struct Adjusted {
+    R rt, rqv, rqc, rqr;
+  };
+  auto adjust = [&](const Lv& cur, int k) -> Adjusted {
     const R rho = rmax(pert ? cur.rho + a.base.rho[k] : cur.rho, R(1.0e-6));
     const R rt0 = pert ? cur.rt + a.base.rt[k] : cur.rt;
-    const R in_qv = cur.qv, in_qc = cur.qc, in_qr = cur.qr;
-    MicroCell<R> m = micro_prepare(rho, rt0, in_qv, in_qc, in_qr);
+    MicroCell<R> m = micro_prepare(rho, rt0, cur.qv, cur.qc, cur.qr);
     const R th0 = m.th;
     micro_apply(m, mc);
-    const R th = m.th, qv = m.qv, qc = m.qc, qr = m.qr;
-    a.qv[c] = rho * qv;
-    a.qc[c] = rho * qc;
-    R rqr = rho * qr;
-    a.rt[c] = pert ? rtp + rho * (th - th0) : rho * th;
+    return {pert ? cur.rt + rho * (m.th - th0) : rho * m.th, rho * m.qv, rho * m.qc, rho * m.qr};
+  };
+  // What stays of a cell's rain, and what it lets fall (into inc).
+  auto fall = [&](R rqr, int k) -> R {
     if (nominal) {
       const R old = rmax(rqr, R(0)) * dz_nom;
       const R out = frac_nom * old;
@@ -322,18 +321,44 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
       rqr = (old - out + inc) * idz;
       inc = out;
     }
-    a.qr[c] = rqr;
+    return rqr;
+  };
+  // The loads of the level three below are issued before the current level's
+  // arithmetic.
+  size_t c = g.cell(i, j, k1 - 1);
+  Lv l1{}, l2{}, l3{}, above{};
+  if (k1 < g.nz) above = load(c + plane);
+  if (k1 > k0) l1 = load(c);
+  if (k1 - 1 > k0) l2 = load(c - plane);
+  if (k1 - 2 > k0) l3 = load(c - 2 * plane);
+  if (nch > 1) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the level above has been read
+    __syncthreads();
+  }
+  if (!in) return;
+  if (k1 < g.nz && (nominal || metric)) fall(adjust(above, k1).rqr, k1);
+  for (int k = k1 - 1; k >= k0; --k) {
+    const Lv cur = l1;
+    l1 = l2;
+    l2 = l3;
+    if (k - 3 >= k0) l3 = load(c - 3 * plane);
+    const Adjusted n = adjust(cur, k);
+    a.qv[c] = n.rqv;
+    a.qc[c] = n.rqc;
+    a.rt[c] = n.rt;
+    a.qr[c] = fall(n.rqr, k);
     c -= plane;
   }
+  if (k0 > 0) return;
   if (nominal || metric) a.precip[static_cast<size_t>(j) * g.nx + i] += inc;
 }
 
 template <class R, bool TERRAIN>
-__global__ void k_warm_rain(WarmRainArgs<R> a) {
+__global__ __launch_bounds__(512) void k_warm_rain(WarmRainArgs<R> a) {
   warm_rain_body<R, TERRAIN>(a, hw_block());
 }
 template <class R, bool TERRAIN>
-__global__ void k_warm_rain_batch(const WarmRainItem<R>* items, BatchMap bm) {
+__global__ __launch_bounds__(512) void k_warm_rain_batch(const WarmRainItem<R>* items, BatchMap bm) {
   VBlock vb;
   const WarmRainItem<R>* it = batch_member(items, bm, vb);
   if (!it) return;
@@ -643,8 +668,16 @@ void launch_rebuild_rt(hipStream_t st, const Geo& g, const R* rho, const R* th, 
 }
 template <class R>
 void launch_warm_rain(hipStream_t st, const WarmRainArgs<R>& a, bool terrain) {
-  const dim3 b(64, 4, 1);
-  const dim3 gr((a.g.nx + 63) / 64, (a.g.ny + 3) / 4);
+  // Enough waves to cover the loads, and no more than that (each chunk costs a
+  // second adjustment of a level): by the number of 64-column waves.  Measured
+  // with 1 / 2 / 4 / 8 chunks (us): 4096 waves of 64 levels in FP32 193, 150,
+  // 158, 177; 1024 in FP64 237, 163, 125, 121; eight members of 192 to 896
+  // waves in one launch 152, 124, 119, 126; 64 waves of 40 levels 38, 22, 13, 10.
+  const dim3 gr((a.g.nx + 63) / 64, a.g.ny);
+  const long waves = static_cast<long>(gr.x) * gr.y;
+  int chunks = waves >= 2048 ? 2 : waves >= 128 ? 4 : 8;
+  while (chunks > 1 && a.g.nz < 4 * chunks) chunks /= 2;
+  const dim3 b(64, chunks, 1);
   if (recorder()) {
     const void* fn = terrain ? reinterpret_cast<const void*>(&k_warm_rain_batch<R, true>)
                              : reinterpret_cast<const void*>(&k_warm_rain_batch<R, false>);
