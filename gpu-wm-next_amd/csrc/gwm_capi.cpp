@@ -394,6 +394,7 @@ struct gwm_state {
   // wrote, ready for the next stage's theta_ref (no pass over the state)
   const void* theta_parts_rho = nullptr;
   int theta_nparts = 0;
+  const double* theta_part = nullptr;
   // view of a stage set; a tracer stage view also points at the stage's
   // tracer buffers (empty: the owner's canonical tracers)
   void* vset[5] = {};
@@ -471,14 +472,15 @@ struct gwm_state {
     return sur_queue;
   }
   // Partial-sum buffer of the step's level means (both uses fit).
-  double* level_part() {
-    if (!step_part) {
-      const Geo& gg = g();
-      const size_t per = std::max<size_t>(gwm::fast_column_parts(gg.nx, gg.ny),
-                                          gwm::level_partials_chunks(gg.ny));
-      step_part = static_cast<double*>(dalloc(static_cast<size_t>(gg.nz) * per * 2 * sizeof(double)));
-    }
-    return step_part;
+  // Two halves: a substep that sums its own level partials reads one while it
+  // writes the next substep's to the other.
+  double* level_part(int half) {
+    const Geo& gg = g();
+    const size_t per = std::max<size_t>(gwm::fast_column_parts(gg.nx, gg.ny),
+                                        gwm::level_partials_chunks(gg.ny));
+    const size_t n = static_cast<size_t>(gg.nz) * per * 2;
+    if (!step_part) step_part = static_cast<double*>(dalloc(2 * n * sizeof(double)));
+    return step_part + (half & 1 ? n : 0);
   }
 };
 
@@ -515,20 +517,35 @@ void ensure_synced(gwm_state* S, void** fs) {
   S->faces_synced = true;
 }
 
+// Level means of small grids are left to the kernels that use them; not in a
+// recorded (batched) step, whose members must launch the same sequence.
+bool inline_parts(const Geo& g, int nparts) {
+  return nparts <= gwm::kInlineParts &&
+         static_cast<long>(g.nx) * g.ny * g.nz <= gwm::kInlineCells && !gwm::recorder();
+}
+
 template <class R>
-void level_theta_ref(gwm_state* S, const R* rho, const R* rt) {
+void level_theta_ref(gwm_state* S, const R* rho, const R* rt, gwm::SlowArgs<R>& a) {
   const Geo& g = S->g();
   if (!S->theta_ref) S->theta_ref = dalloc(g.nz * sizeof(R));
-  double* part = S->level_part();
+  a.theta_ref = static_cast<const R*>(S->theta_ref);
+  const double* part = nullptr;
   int nch = 0;
   if (S->theta_parts_rho == rho) {  // emitted by the subcycle that wrote (rho, rt)
     nch = S->theta_nparts;
+    part = S->theta_part;
   } else {
     Timed t(S->ctx, "level_partials");
-    gwm::launch_level_partials<R>(S->ctx->stream, g, rho, rt, 0, part, &nch, S->base<R>());
+    double* p = S->level_part(0);
+    gwm::launch_level_partials<R>(S->ctx->stream, g, rho, rt, 0, p, &nch, S->base<R>());
+    part = p;
   }
   S->theta_parts_rho = nullptr;
-  {
+  if (!S->grid->terrain_nonzero && inline_parts(g, nch)) {
+    a.th_part = part;
+    a.th_nparts = nch;
+    a.th_count = static_cast<double>(g.nx) * g.ny;
+  } else {
     Timed t(S->ctx, "level_finalize");
     gwm::launch_level_finalize<R>(S->ctx->stream, g.nz, nch, part, 0,
                                   static_cast<double>(g.nx) * g.ny,
@@ -621,22 +638,30 @@ int subcycle(gwm_state* S, const gwm_step_config& c, const R* rho_in, const R* t
   int last = z0;
   // Level partials: substep 0 from a pass over the entry state, later
   // substeps from the previous substep's column kernel.
-  double* part = flat ? S->level_part() : nullptr;
   int nparts = 0;
+  const bool means_inline = !G->terrain_nonzero;  // (the flat march sums few partials itself)
   for (int s = 0; s < ns; ++s) {
     const int o = outs[s % 2];
+    gwm::FastArgs<R> a{};
+    double* part = flat ? S->level_part(s + 1) : nullptr;  // the next substep's
     if (flat) {
+      double* here = S->level_part(s);
       if (s == 0) {
         Timed t(S->ctx, "level_partials");
-        gwm::launch_level_partials<R>(S->ctx->stream, g, rho, theta, 1, part, &nparts,
+        gwm::launch_level_partials<R>(S->ctx->stream, g, rho, theta, 1, here, &nparts,
                                       S->base<R>());
       }
-      Timed t(S->ctx, "level_finalize");
-      gwm::launch_level_finalize<R>(S->ctx->stream, g.nz, nparts, part, 1,
-                                    static_cast<double>(g.nx) * g.ny,
-                                    static_cast<R*>(S->rref_lev), static_cast<R*>(S->pref_lev));
+      const double count = static_cast<double>(g.nx) * g.ny;
+      if (means_inline && inline_parts(g, nparts)) {
+        a.lev_part = here;
+        a.lev_nparts = nparts;
+        a.lev_inv = R(1) / static_cast<R>(count);
+      } else {
+        Timed t(S->ctx, "level_finalize");
+        gwm::launch_level_finalize<R>(S->ctx->stream, g.nz, nparts, here, 1, count,
+                                      static_cast<R*>(S->rref_lev), static_cast<R*>(S->pref_lev));
+      }
     }
-    gwm::FastArgs<R> a{};
     a.g = g;
     a.rho = rho;
     a.theta = theta;
@@ -691,6 +716,7 @@ int subcycle(gwm_state* S, const gwm_step_config& c, const R* rho_in, const R* t
     if (emit_th) {
       S->theta_parts_rho = a.rho_out;
       S->theta_nparts = nparts;
+      S->theta_part = part;
     }
   }
   return last;
@@ -700,14 +726,13 @@ template <class R>
 void slow_stage(gwm_state* S, const gwm_step_config& c, void* const* in, void* const* q0,
                 void* const* out, int mode, R wa, R wb, int out_theta) {
   const Geo& g = S->g();
-  level_theta_ref<R>(S, static_cast<const R*>(in[0]), static_cast<const R*>(in[1]));
   gwm::SlowArgs<R> a{};
+  level_theta_ref<R>(S, static_cast<const R*>(in[0]), static_cast<const R*>(in[1]), a);
   a.g = g;
   a.s = dstate<R>(in);
   if (q0) a.q0 = dstate<R>(q0);
   a.out = dstate<R>(out);
   a.m = S->grid->dm<R>();
-  a.theta_ref = static_cast<const R*>(S->theta_ref);
   a.gravity = static_cast<R>(c.gravity);
   a.dt = static_cast<R>(c.dt);
   a.wa = wa;

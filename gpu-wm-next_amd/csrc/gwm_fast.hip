@@ -91,7 +91,7 @@ __device__ __forceinline__ void emit_part(const FastArgs<R>& a, double* part_out
 // so that a substep reads first the levels the previous substep, marching
 // up, wrote last; every cell's arithmetic is the upward march's, in the
 // same order, so the results are identical.
-template <class R, bool PERT, int KIND, int TYV, bool DOWN>
+template <class R, bool PERT, int KIND, int TYV, bool DOWN, bool SUMS>
 __device__ __forceinline__ void fast_body(const FastArgs<R>& a, int tiles_x, int tiles, int nkc,
                                           double* part_out, const VBlock& vb) {
   constexpr int TY = TYV, PY = TY + 2, PN = PX * PY;
@@ -134,8 +134,10 @@ __device__ __forceinline__ void fast_body(const FastArgs<R>& a, int tiles_x, int
     const int kk = k0 - 1 + q;
     const int kc = kk < 0 ? 0 : (kk >= nz ? nz - 1 : kk), kf = kk < 0 ? 0 : (kk > nz ? nz : kk);
     R* e = lev + q * NLV;
-    e[LV_PREF] = a.pref_lev[kc];
-    e[LV_RREF] = a.rref_lev[kc];
+    if constexpr (!SUMS) {
+      e[LV_PREF] = a.pref_lev[kc];
+      e[LV_RREF] = a.rref_lev[kc];
+    }
     e[LV_IDZF] = a.m.lev_idz_f[kf];
     e[LV_IDZC] = a.m.lev_idz_c[kc];
     if (PERT) {
@@ -143,6 +145,18 @@ __device__ __forceinline__ void fast_body(const FastArgs<R>& a, int tiles_x, int
       e[LV_BTH] = a.base.th[kc];
       e[LV_BRT] = a.base.rt[kc];
       e[LV_BP] = a.base.p[kc];
+    }
+  }
+  if constexpr (SUMS) {  // level means, one level per wave
+#pragma unroll 2
+    for (int q = ly; q < k1 - k0 + 3; q += TY) {
+      const int kk = k0 - 1 + q;
+      double s0, s1;
+      level_sums(a.lev_part, a.lev_nparts, kk < 0 ? 0 : (kk >= nz ? nz - 1 : kk), lx, s0, s1);
+      if (lx == 63) {
+        lev[q * NLV + LV_RREF] = static_cast<R>(s0) * a.lev_inv;
+        lev[q * NLV + LV_PREF] = static_cast<R>(s1) * a.lev_inv;
+      }
     }
   }
   auto LV = [&](int kk, int q) -> R { return lev[(kk - k0 + 1) * NLV + q]; };
@@ -938,20 +952,22 @@ void launch_column_reference(hipStream_t st, const FastArgs<R>& a) {
 }
 
 // FORM: 0 full and 1 perturbation form on flat grids, marching up; 2 and 3 the
-// same marching down; 4 + REF on terrain.
-template <class R, int FORM, int KIND, int TYV>
+// same marching down; 4 + REF on terrain.  SUMS: the level means are summed
+// from their partials in the prologue (a kernel of its own: the branch in the
+// common one cost substeps that do not take it 1.5 %).
+template <class R, int FORM, int KIND, int TYV, bool SUMS>
 __device__ __forceinline__ void fast_form(const FastArgs<R>& a, int tiles_x, int tiles, int nkc,
                                           double* part_out, const VBlock& vb) {
   if constexpr (FORM >= 4)
     fast_terrain_body<R, FORM - 4, KIND, TYV>(a, tiles_x, tiles, nkc, part_out, vb);
   else
-    fast_body<R, (FORM & 1) != 0, KIND, TYV, (FORM & 2) != 0>(a, tiles_x, tiles, nkc, part_out, vb);
+    fast_body<R, (FORM & 1) != 0, KIND, TYV, (FORM & 2) != 0, SUMS>(a, tiles_x, tiles, nkc, part_out, vb);
 }
 
-template <class R, int FORM, int KIND, int TYV>
+template <class R, int FORM, int KIND, int TYV, bool SUMS>
 __global__ __launch_bounds__(TX * TYV) void k_fast_column(FastArgs<R> a, int tiles_x, int tiles,
                                                           int nkc, double* part_out) {
-  fast_form<R, FORM, KIND, TYV>(a, tiles_x, tiles, nkc, part_out, hw_block());
+  fast_form<R, FORM, KIND, TYV, SUMS>(a, tiles_x, tiles, nkc, part_out, hw_block());
 }
 template <class R, int FORM, int KIND, int TYV>
 __global__ __launch_bounds__(TX * TYV) void k_fast_column_batch(
@@ -961,7 +977,7 @@ __global__ __launch_bounds__(TX * TYV) void k_fast_column_batch(
   if (!it) return;
   // the member's arguments, read once before the kernel stores anything
   const FastArgs<R> a = it->a;
-  fast_form<R, FORM, KIND, TYV>(a, it->tiles_x, it->tiles, it->nkc, it->part_out, vb);
+  fast_form<R, FORM, KIND, TYV, false>(a, it->tiles_x, it->tiles, it->nkc, it->part_out, vb);
 }
 
 template <class R, int FORM, int TYV>
@@ -981,23 +997,25 @@ void launch_fast_kind(hipStream_t st, const FastArgs<R>& a, int nkc, double* par
                   static_cast<int>(grid.x), 1);
     return;
   }
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, blk, lds, st, a, tx, tiles, nkc, part_out);
+  };
+  if constexpr (FORM < 4) {
+    if (a.lev_part) {
+      switch (kind) {
+        case 0: go(k_fast_column<R, FORM, 0, TYV, true>); break;
+        case 1: go(k_fast_column<R, FORM, 1, TYV, true>); break;
+        case 2: go(k_fast_column<R, FORM, 2, TYV, true>); break;
+        default: go(k_fast_column<R, FORM, 3, TYV, true>); break;
+      }
+      return;
+    }
+  }
   switch (kind) {
-    case 0:
-      hipLaunchKernelGGL((k_fast_column<R, FORM, 0, TYV>), grid, blk, lds, st, a, tx, tiles, nkc,
-                         part_out);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_fast_column<R, FORM, 1, TYV>), grid, blk, lds, st, a, tx, tiles, nkc,
-                         part_out);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_fast_column<R, FORM, 2, TYV>), grid, blk, lds, st, a, tx, tiles, nkc,
-                         part_out);
-      break;
-    default:
-      hipLaunchKernelGGL((k_fast_column<R, FORM, 3, TYV>), grid, blk, lds, st, a, tx, tiles, nkc,
-                         part_out);
-      break;
+    case 0: go(k_fast_column<R, FORM, 0, TYV, false>); break;
+    case 1: go(k_fast_column<R, FORM, 1, TYV, false>); break;
+    case 2: go(k_fast_column<R, FORM, 2, TYV, false>); break;
+    default: go(k_fast_column<R, FORM, 3, TYV, false>); break;
   }
 }
 

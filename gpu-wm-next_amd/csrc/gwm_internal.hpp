@@ -582,6 +582,18 @@ __device__ inline float wave_sum_to63(float v) {
   return v;
 }
 
+// Sums of one level's partials p[k][n][2], n <= 128, by a whole wave: complete
+// in lane 63, in the order of k_level_finalize.
+__device__ inline void level_sums(const double* p, int n, int k, int lane, double& s0, double& s1) {
+  typedef const __attribute__((address_space(1))) double gd;
+  gd* q = (gd*)p + 2 * static_cast<size_t>(k) * n;
+  const bool a = lane < n, b = lane + 64 < n;
+  const double x0 = a ? q[2 * lane] : 0.0, x1 = a ? q[2 * lane + 1] : 0.0;
+  const double y0 = b ? q[2 * lane + 128] : 0.0, y1 = b ? q[2 * lane + 129] : 0.0;
+  s0 = wave_sum_to63(x0) + wave_sum_to63(y0);
+  s1 = wave_sum_to63(x1) + wave_sum_to63(y1);
+}
+
 // Element offsets (level 0) of one staged position (ii, jj) of a tile: its
 // cell (and z-faces), x-faces ii and ii+1, y-faces jj and jj+1, with the 1x1
 // halo map applied once; -1 marks a value that is zero (open side).

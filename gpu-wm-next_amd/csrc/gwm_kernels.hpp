@@ -16,6 +16,11 @@ struct SlowArgs {
   DState<R> out;  // output (tendencies in mode 0)
   DMetrics<R> m;
   const R* theta_ref;  // nz
+  // theta_ref's level partials, summed by the work-groups themselves (set:
+  // theta_ref is not read; flat grids), how many a level has, and the cells of a level
+  const double* th_part;
+  int th_nparts;
+  double th_count;
   R gravity;
   R dt;
   R wa, wb;
@@ -36,6 +41,12 @@ struct FastArgs {
   R *rho_out, *u_out, *v_out, *w_out;  // face departures, full faces if last
   R* rt_out;  // rho*theta rebuild (last substep), may be null
   const R *rref_lev, *pref_lev;  // flat reference (nz)
+  // the level partials of rref_lev and pref_lev, summed by the work-groups
+  // themselves (set: those are not read), how many a level has, and
+  // 1 / cells of a level
+  const double* lev_part;
+  int lev_nparts;
+  R lev_inv;
   R *rref3, *pref3;  // column reference (metric layout; col_ref), scratch of the launch
   DMetrics<R> m;
   R dtf, gravity;
@@ -105,6 +116,15 @@ struct BudgetArgs {
 template <class R>
 void launch_level_partials(hipStream_t st, const Geo& g, const R* rho, const R* aux, int mode,
                            double* partials, int* nchunk_out, Base<R> base = Base<R>{});
+// Up to this many partials a level (two a lane) and cells, the kernels that
+// use a level's mean sum them in their prologue (level_sums) instead of a
+// launch that does so for all of them: a launch costs 4 to 5 us, the prologue
+// about one in every round of work-groups, and a million cells are one round.
+// Same bits either way.  Four captured moist steps of 64 x 64 x 40: 950 -> 876
+// us; a slow tendency call of 500 x 380 x 60, whose 48 partials a level would
+// pass, lost 5 % with it.
+constexpr int kInlineParts = 128;
+constexpr long kInlineCells = 1L << 20;
 // Partials per level written by launch_level_partials for ny rows.
 int level_partials_chunks(int ny);
 template <class R>

@@ -61,7 +61,10 @@ __device__ inline R upwind(R a, R ql, R qr) {  // dry_momentum_flux.cu:75-77
 // work-group.
 enum { SL_TREF = 0, SL_IDZF, SL_IDZC, SL_BRHO, SL_BTH, SL_BRT, SL_BP, SL_N };
 
-template <class R, bool TERRAIN, bool PERT, int MODE>
+// SUMS: theta's level means are summed from their partials in the prologue (a
+// kernel of its own: the branch in the common one cost stages that do not take
+// it 2 %).
+template <class R, bool TERRAIN, bool PERT, int MODE, bool SUMS>
 __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int tiles, int nkc,
                                           const VBlock& vb) {
   // FP32 also stages the raw face momenta of each level (tile plus ring), so
@@ -132,7 +135,7 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
     const int kk = k0 - 1 + q;
     const int kc = kk < 0 ? 0 : (kk >= nz ? nz - 1 : kk), kf = kk < 0 ? 0 : (kk > nz ? nz : kk);
     R* e = lev + q * SL_N;
-    e[SL_TREF] = a.theta_ref[kc];
+    if constexpr (!SUMS) e[SL_TREF] = a.theta_ref[kc];
     if (!TERRAIN) {
       e[SL_IDZF] = a.m.lev_idz_f[kf];
       e[SL_IDZC] = a.m.lev_idz_c[kc];
@@ -142,6 +145,15 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
       e[SL_BTH] = a.base.th[kc];
       e[SL_BRT] = a.base.rt[kc];
       e[SL_BP] = a.base.p[kc];
+    }
+  }
+  if constexpr (SUMS) {  // level means of theta, one level per wave
+#pragma unroll 2
+    for (int q = ly; q < k1 - k0 + 3; q += TY) {
+      const int kk = k0 - 1 + q;
+      double s0, s1;
+      level_sums(a.th_part, a.th_nparts, kk < 0 ? 0 : (kk >= nz ? nz - 1 : kk), lx, s0, s1);
+      if (lx == 63) lev[q * SL_N + SL_TREF] = static_cast<R>(s0 / a.th_count);
     }
   }
   auto LV = [&](int kk, int q) -> R { return lev[(kk - k0 + 1) * SL_N + q]; };
@@ -715,10 +727,10 @@ __device__ __forceinline__ void slow_body(const SlowArgs<R>& a, int tiles_x, int
   }
 }
 
-template <class R, bool TERRAIN, bool PERT, int MODE>
+template <class R, bool TERRAIN, bool PERT, int MODE, bool SUMS>
 __global__ __launch_bounds__(TX * TY) void k_slow_column(SlowArgs<R> a, int tiles_x, int tiles,
                                                          int nkc) {
-  slow_body<R, TERRAIN, PERT, MODE>(a, tiles_x, tiles, nkc, hw_block());
+  slow_body<R, TERRAIN, PERT, MODE, SUMS>(a, tiles_x, tiles, nkc, hw_block());
 }
 template <class R, bool TERRAIN, bool PERT, int MODE>
 __global__ __launch_bounds__(TX * TY) void k_slow_column_batch(
@@ -728,7 +740,7 @@ __global__ __launch_bounds__(TX * TY) void k_slow_column_batch(
   if (!it) return;
   // the member's arguments, read once before the kernel stores anything
   const SlowArgs<R> a = it->a;
-  slow_body<R, TERRAIN, PERT, MODE>(a, it->tiles_x, it->tiles, it->nkc, vb);
+  slow_body<R, TERRAIN, PERT, MODE, false>(a, it->tiles_x, it->tiles, it->nkc, vb);
 }
 
 template <class R, bool TERRAIN, bool PERT>
@@ -742,19 +754,21 @@ void launch_slow_mode(hipStream_t st, const SlowArgs<R>& a, dim3 grid, dim3 blk,
     record_launch(fn, blk, lds, SlowItem<R>{a, tx, tiles, nkc, 0, 0}, static_cast<int>(grid.x), 1);
     return;
   }
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, lds, st, a, tx, tiles, nkc); };
+  if constexpr (!TERRAIN) {
+    if (a.th_part) {
+      switch (a.mode) {
+        case 0: go(k_slow_column<R, TERRAIN, PERT, 0, true>); break;
+        case 1: go(k_slow_column<R, TERRAIN, PERT, 1, true>); break;
+        default: go(k_slow_column<R, TERRAIN, PERT, 2, true>); break;
+      }
+      return;
+    }
+  }
   switch (a.mode) {
-    case 0:
-      hipLaunchKernelGGL((k_slow_column<R, TERRAIN, PERT, 0>), grid, blk, lds, st, a, tx, tiles,
-                         nkc);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_slow_column<R, TERRAIN, PERT, 1>), grid, blk, lds, st, a, tx, tiles,
-                         nkc);
-      break;
-    default:
-      hipLaunchKernelGGL((k_slow_column<R, TERRAIN, PERT, 2>), grid, blk, lds, st, a, tx, tiles,
-                         nkc);
-      break;
+    case 0: go(k_slow_column<R, TERRAIN, PERT, 0, false>); break;
+    case 1: go(k_slow_column<R, TERRAIN, PERT, 1, false>); break;
+    default: go(k_slow_column<R, TERRAIN, PERT, 2, false>); break;
   }
 }
 
