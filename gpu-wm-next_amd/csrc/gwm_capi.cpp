@@ -2238,14 +2238,15 @@ int gwm_state_copy(gwm_state* dst, const gwm_state* src) {
       dst->base_rt64 = src->base_rt64;
       push_base(dst);
     }
-    for (int f = 0; f < 5; ++f)
-      HIPCHK(hipMemcpyAsync(dst->field(f), s->field(f), s->fsize(f) * s->es(),
-                            hipMemcpyDeviceToDevice, dst->ctx->stream));
+    gwm::CopyJobs jobs;
+    for (int f = 0; f < 5; ++f) jobs.add(dst->field(f), s->field(f), s->fsize(f) * s->es());
     for (int t = 0; t < s->ntr; ++t)
-      HIPCHK(hipMemcpyAsync(dst->field(GWM_TRACER0 + t), s->field(GWM_TRACER0 + t),
-                            s->fsize(GWM_RHO) * s->es(), hipMemcpyDeviceToDevice, dst->ctx->stream));
-    HIPCHK(hipMemcpyAsync(dst->precip, s->precip, s->fsize(GWM_PRECIP) * s->es(),
-                          hipMemcpyDeviceToDevice, dst->ctx->stream));
+      jobs.add(dst->field(GWM_TRACER0 + t), s->field(GWM_TRACER0 + t), s->fsize(GWM_RHO) * s->es());
+    jobs.add(dst->precip, s->precip, s->fsize(GWM_PRECIP) * s->es());
+    for (int q = 0; q < jobs.n; ++q)  // (a stage view has no bucket of its own)
+      require(jobs.src[q] && jobs.dst[q], "state copy: a field is not allocated");
+    gwm::launch_copy_jobs(dst->ctx->stream, jobs);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(dst->ctx->stream));
     dst->faces_synced = s->faces_synced;
   });

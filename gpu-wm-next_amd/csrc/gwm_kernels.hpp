@@ -223,6 +223,22 @@ void launch_metrics(hipStream_t st, const Geo& g, const double* zif, const doubl
                     R* idz_c, R* idz_f, R* sx, R* sy, R* terr);
 template <class R>
 void launch_copy(hipStream_t st, const R* src, R* dst, size_t n);
+// Copies of several buffers (whole 4-byte words, not overlapping or the same)
+// in one launch.
+constexpr int kCopyJobs = 6 + kMaxTracers;
+struct CopyJobs {
+  const void* src[kCopyJobs];
+  void* dst[kCopyJobs];
+  size_t words[kCopyJobs];
+  unsigned chunk0[kCopyJobs + 1];  // filled by the launcher
+  int n = 0;
+  void add(void* d, const void* s, size_t bytes) {
+    src[n] = s;
+    dst[n] = d;
+    words[n++] = bytes / 4;
+  }
+};
+void launch_copy_jobs(hipStream_t st, CopyJobs j);
 template <class R>
 void launch_fill(hipStream_t st, R* dst, size_t n, R v);
 
