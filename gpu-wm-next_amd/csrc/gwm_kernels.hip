@@ -355,7 +355,10 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
 
 template <class R, bool TERRAIN>
 __global__ __launch_bounds__(512) void k_warm_rain(WarmRainArgs<R> a) {
-  warm_rain_body<R, TERRAIN>(a, hw_block());
+  // (a row of 64-column waves after the other in x: the launch's y extent
+  // would limit the rows)
+  const int gx = (a.g.nx + 63) / 64, b = static_cast<int>(blockIdx.x);
+  warm_rain_body<R, TERRAIN>(a, VBlock{b % gx, b / gx, gx, a.g.ny});
 }
 template <class R, bool TERRAIN>
 __global__ __launch_bounds__(512) void k_warm_rain_batch(const WarmRainItem<R>* items, BatchMap bm) {
@@ -715,10 +718,11 @@ void launch_warm_rain(hipStream_t st, const WarmRainArgs<R>& a, bool terrain) {
                   static_cast<int>(gr.y));
     return;
   }
+  const dim3 flat(gr.x * gr.y);
   if (terrain)
-    hipLaunchKernelGGL((k_warm_rain<R, true>), gr, b, 0, st, a);
+    hipLaunchKernelGGL((k_warm_rain<R, true>), flat, b, 0, st, a);
   else
-    hipLaunchKernelGGL((k_warm_rain<R, false>), gr, b, 0, st, a);
+    hipLaunchKernelGGL((k_warm_rain<R, false>), flat, b, 0, st, a);
 }
 template <class R>
 void launch_halo_fill(hipStream_t st, const Geo& g, int orient, R* f) {

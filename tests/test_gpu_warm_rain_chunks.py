@@ -27,7 +27,7 @@ def test_chunk_counts_agree(nz, prec, metric):
     f = {k: v.astype(ctx.dtype) for k, v in f.items()}
     cfg = dict(dt=5.0, rain_terminal_velocity=12.0, sedimentation_layer_depth_m=400.0)
     first = None
-    for rows in (ny, 256, 2048):
+    for rows in (ny, 256, 2048) + ((65600,) if nz == 1 else ()):
         st = G.State(G.Grid(ctx, nx, rows, nz, z_interfaces=zi), 3)
         for k, v in f.items():
             st.set(k, np.tile(v, (1, rows // ny, 1)))
