@@ -825,11 +825,11 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
     const R dz = ld32(a.m.zc, m) - ld32(a.m.zc, m - n2);
     const R pa = q_pressure(r, r * th);
     // away from the floors of rho, p, p / p0 and R_d theta Exner, each with
-    // room for the series' range; else u is out of range and the power is taken
+    // room for the series' range; else u is NaN and the power is taken
     const bool series = r >= R(2.0e-6) && pa >= R(2) && pa >= R(2.0e-6) * r;
     const int q = k % kRefSeg;
-    s_pa[buf][q][lane] = series ? pa : R(-1);
-    s_ra[buf][q][lane] = series ? qrcp(pa) : R(1);
+    s_pa[buf][q][lane] = pa;
+    s_ra[buf][q][lane] = series ? qrcp(pa) : static_cast<R>(__builtin_nanf(""));
     s_rho[buf][q][lane] = r;
     s_h[buf][q][lane] = grav * R(0.5) * dz;
   };
@@ -874,9 +874,11 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
         nx = prep(k + 1 < ke ? k + 1 : k);  // in flight during this level
         // p_{k+1} less the layer's weight, in one rounding
         auto weigh = [&](R sum) -> R { return static_cast<R>(fma(-c.h, sum, p)); };
-        R far = R(0);
+        // (a NaN is not near: no series at this level, an infinite pressure,
+        // or an overflow on the way)
+        bool near = true;
         auto shape = [&](R u) -> R {  // rho(pa (1 + u)) / rho
-          far = rmax(far, u < R(0) ? -u : u);
+          near &= (u < R(0) ? -u : u) <= R(0.03125);
           return rho_series(u);
         };
         R pn = R(0), rn = R(0), left = R(0);
@@ -899,7 +901,7 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
         }
         settle(static_cast<R>(fma(c.rho, f, r)));
         rn = c.rho * shape((pn - c.pa) * c.ra);
-        if (!(far <= R(0.03125))) {
+        if (!near) {
           const R th = q_theta(c.rho, c.rho * ld32(a.theta, c0 + static_cast<unsigned>(k) * pc));
           R sum = r + r;
           pn = rmax(weigh(sum), R(1));

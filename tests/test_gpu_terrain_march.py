@@ -47,3 +47,48 @@ def test_terrain_substeps_against_oracle(nx, ny, nz, z_top, open_x, thin):
             # dt / d over three substeps, relative to the field's own size
             scale = np.abs(want).max() + 1.0
             assert np.abs(v - want).max() <= 2e-11 * scale, (f, code)
+
+
+@pytest.mark.parametrize("prec", [G.F64, G.F32])
+@pytest.mark.parametrize("case", ["overflow", "thin"])
+def test_column_reference_outside_the_series(prec, case):
+    """Levels where the density series does not hold.  A cell whose pressure
+    overflows (its theta is finite, so the power gives the reference a finite
+    density there): w is not finite on the cell's two faces only.  Pressures
+    between one and two Pascal (too near the floor of one Pascal), with layers
+    whose weight the series' variable would take for a small departure: the
+    reference ends on the floor.  Against the oracle of the same precision;
+    each p carries a few roundings on both sides, so p - p_ref of a face is off
+    by at most 16 of them (the floored case is exact in p_ref)."""
+    nx, ny, nz = 70, 6, 9
+    if case == "thin":
+        theta, p = 300.0, 1.5
+        rho0 = p / (287.05 * theta * (p / 1e5) ** 0.2854)
+        z_top = nz * (p + 1.0) / (9.81 * rho0)
+    else:
+        theta, rho0, z_top = 300.0, 1.0, 9000.0
+    kw = dict(z_top=z_top, terrain=G.cosine_mountain(nx, ny, 0.001 * z_top))
+    cfg = dict(dt=0.2, fast_substeps=1)
+    w = O.World(nx, ny, nz, precision=8 if prec == G.F64 else 4, **kw)
+    ctx = G.Context(0, prec)
+    rho = np.full((nz, ny, nx), rho0)
+    rt = rho * theta
+    if case == "overflow":
+        rt[4, 3, 65] = 1e30 if prec == G.F32 else 1e250
+    st = G.State(G.Grid(ctx, nx, ny, nz, **kw), 0)
+    for f, v in ((O.RHO, rho), (O.RHO_THETA, rt), (O.MOM_U, 0.0), (O.MOM_V, 0.0), (O.MOM_W, 0.0)):
+        v = np.broadcast_to(v, w.get(f).shape).astype(ctx.dtype)
+        w.set(f, v.astype(w.get(f).dtype))
+        st.set(f, v)
+    w.fast_modes(O.step_cfg(**cfg))
+    st.fast_modes(G.step_config(**cfg))
+    got, want = st.get(O.MOM_W), w.get(O.MOM_W)
+    faces = np.isfinite(got)
+    if case == "overflow":
+        assert not faces[4:6, 3, 65].any() and faces.sum() == faces.size - 2
+    else:
+        assert faces.all()
+    p_max = 1.3e5 if case == "overflow" else 1.5
+    bound = 0.2 * nz / z_top * 1.01 * 16 * np.finfo(ctx.dtype).eps * p_max
+    err = np.abs(got[faces] - want[faces]).max()
+    assert err <= bound + 4 * np.finfo(ctx.dtype).eps * np.abs(want[faces]).max()
