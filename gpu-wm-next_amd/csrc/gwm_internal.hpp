@@ -292,13 +292,15 @@ __device__ inline R q_theta(R rho, R rt) {
 // its roundings, which the FP32 oracle has too.  FP64: theta = (rho theta) /
 // max(rho, 1e-6), so the density cancels except below its floor, and the ratio
 // is two products instead of two divisions and two products (with fewer
-// roundings).
+// roundings).  A density that is infinite or NaN does not cancel (theta is
+// zero or NaN, the ratio NaN): the ratio takes its floor, as in FP32.
 __device__ inline float q_eos_ratio(float rho, float rt) {
   return rmax(qdiv(rho * Phys<float>::Rd * q_theta(rho, rt), Phys<float>::p0), 1.0e-6f);
 }
 __device__ inline double q_eos_ratio(double rho, double rt) {
   constexpr double c = Phys<double>::Rd / Phys<double>::p0;
-  return rmax(rt * c * rmin(rho * 1.0e6, 1.0), 1.0e-6);
+  const double thin = rho < __builtin_inf() ? rmin(rho * 1.0e6, 1.0) : 0.0;
+  return rmax(rt * c * thin, 1.0e-6);
 }
 template <class R>
 __device__ inline R q_pressure(R rho, R rt) {

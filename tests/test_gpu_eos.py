@@ -44,3 +44,30 @@ def test_pressure_of_the_step_kernels(prec, thin):
     want = (left - p) / 1000
     bound = 6 * eps * (np.abs(p) + np.abs(left)) / 1000 + 2 * eps * np.abs(want)
     assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / bound).max())
+
+
+def test_fp64_pressure_of_a_state_that_is_not_finite():
+    """A density that is infinite or NaN makes the ratio NaN, which takes the
+    floor (p0 1e-6^gamma), whatever rho theta is; so do a NaN and a negative
+    infinity of rho theta.  Through the slow tendency of u at rest, on the
+    faces beside the cell: its other terms are zero."""
+    nx, ny, nz = 66, 12, 3
+    ctx = G.Context(0, G.F64)
+    grid = G.Grid(ctx, nx, ny, nz, z_interfaces=np.linspace(0.0, 900.0, nz + 1))
+    st = G.State(grid, 0)
+    rho, rt = np.full((nz, ny, nx), 1.1), np.full((nz, ny, nx), 330.0)
+    inf, nan = np.inf, np.nan
+    cells = [(inf, 330.0), (-inf, 330.0), (nan, 330.0), (inf, inf), (nan, inf), (inf, 0.0),
+             (inf, nan), (1.1, nan), (1.1, -inf)]
+    for j, (r, t) in enumerate(cells):
+        rho[1, j, 64], rt[1, j, 64] = r, t
+    st.set(0, rho.astype(ctx.dtype))
+    st.set(1, rt.astype(ctx.dtype))
+    st.slow_tendencies(G.step_config(1.0, 1))
+    du = st.get(8)[1].astype(np.float64)
+    p = 1e5 * (330.0 * 287.05 / 1e5) ** (1.0 / (1.0 - 0.2854))
+    p_floor = 1e5 * 1e-6 ** (1.0 / (1.0 - 0.2854))
+    bound = 12 * 2.0 ** -52 * p / 1000  # six roundings of p, the kernel's and numpy's
+    for j, cell in enumerate(cells):
+        assert abs(du[j, 64] - (p - p_floor) / 1000) <= bound, cell
+        assert abs(du[j, 65] - (p_floor - p) / 1000) <= bound, cell
