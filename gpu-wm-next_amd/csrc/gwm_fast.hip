@@ -768,9 +768,9 @@ __device__ __forceinline__ void fast_terrain_body(const FastArgs<R>& a, int tile
 // FP32; a level with a trial further out, or a state on one of the EOS's
 // floors, is done with the power.  p_a and 1 / p_a do not depend on the chain:
 // wave 0 of a work-group marches 64 columns, and the other seven prepare the
-// next seven levels, one each, in LDS meanwhile.  The roundings of p are
-// carried along (p_lo): p and rho are off by 0.82 and 0.80 epsilon rms in
-// FP64 at 45 levels (plain sums 1.54 and 1.19).
+// next seven levels, one each, in LDS meanwhile.  p_{k+1} is rounded once from
+// p_k: K14 takes the difference of neighbouring levels, which then holds that
+// one rounding (a compensated sum holds two, its levels being rounded apart).
 // ===========================================================================
 constexpr int kRefWaves = 8, kRefSeg = kRefWaves - 1;
 
@@ -839,8 +839,7 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
     const int k = s * kRefSeg + wave - 1;
     if (k >= 1 && k < nz) fill(k, s & 1);
   };
-  // p_lo: what the roundings of p left out so far, added back once it counts
-  R p = R(0), p_lo = R(0), r = R(0);
+  R p = R(0), r = R(0);
   if (wave > 0) {
     fill_seg(0);
   } else {
@@ -881,14 +880,6 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
           near &= (u < R(0) ? -u : u) <= R(0.03125);
           return rho_series(u);
         };
-        R pn = R(0), rn = R(0), left = R(0);
-        // p_{k+1} and what its rounding and those below it left out
-        auto settle = [&](R sum) {
-          const R q = weigh(sum);
-          left = static_cast<R>(fma(-c.h, sum, p - q)) + p_lo;
-          pn = q + left;
-          left -= pn - q;
-        };
         // the trials run in u: the recurrence p - h (r + rho f(u)) is u =
         // (p - pa) / pa - h (r + rho f(u)) / pa
         const R u0 = (p - c.pa) * c.ra, hr = c.h * c.ra;
@@ -899,22 +890,15 @@ __device__ __forceinline__ void column_reference_body(const FastArgs<R>& a, cons
           f = shape(u);
           if (it < 3) u = static_cast<R>(fma(-A, f, B));
         }
-        settle(static_cast<R>(fma(c.rho, f, r)));
-        rn = c.rho * shape((pn - c.pa) * c.ra);
+        R pn = weigh(static_cast<R>(fma(c.rho, f, r)));
+        R rn = c.rho * shape((pn - c.pa) * c.ra);
         if (!near) {
           const R th = q_theta(c.rho, c.rho * ld32(a.theta, c0 + static_cast<unsigned>(k) * pc));
-          R sum = r + r;
-          pn = rmax(weigh(sum), R(1));
+          pn = rmax(weigh(r + r), R(1));
 #pragma unroll 1
-          for (int it = 0; it < 4; ++it) {
-            sum = r + q_rho_from_p_theta(pn, th);
-            pn = rmax(weigh(sum), R(1));
-          }
-          if (pn > R(1)) settle(sum);
-          else left = R(0);
+          for (int it = 0; it < 4; ++it) pn = rmax(weigh(r + q_rho_from_p_theta(pn, th)), R(1));
           rn = q_rho_from_p_theta(pn, th);
         }
-        p_lo = left;
         p = pn;
         r = rn;
         if (in) {

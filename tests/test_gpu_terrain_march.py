@@ -92,3 +92,44 @@ def test_column_reference_outside_the_series(prec, case):
     bound = 0.2 * nz / z_top * 1.01 * 16 * np.finfo(ctx.dtype).eps * p_max
     err = np.abs(got[faces] - want[faces]).max()
     assert err <= bound + 4 * np.finfo(ctx.dtype).eps * np.abs(want[faces]).max()
+
+
+@pytest.mark.parametrize("prec", [G.F64, G.F32])
+def test_reference_differences_hold_one_rounding(prec):
+    """K14 takes differences of the column reference between neighbouring
+    levels; each holds one rounding, that of the upper level's pressure.  All
+    cells share one state, so p cancels from w but for the start of the
+    reference, and the layers are thin: the rounding (half an ulp of 1e5, over
+    dz) outweighs the others, which are relative to the layer's 60 Pa."""
+    nx, ny, nz = 70, 9, 40
+    z_top, dt = 200.0, 0.5
+    ctx = G.Context(0, prec)
+    R, ld = ctx.dtype, np.longdouble
+    kw = dict(z_top=z_top, terrain=G.cosine_mountain(nx, ny, 10.0))
+    grid = G.Grid(ctx, nx, ny, nz, **kw)
+    st = G.State(grid, 0)
+    for f, v in ((O.RHO, 1.16), (O.RHO_THETA, 1.16 * 300.0), (O.MOM_U, 0.0), (O.MOM_V, 0.0),
+                 (O.MOM_W, 0.0)):
+        st.fill(f, v)
+    st.fast_modes(G.step_config(dt=dt, fast_substeps=1))
+    rho, th = ld(R(1.16)), ld(R(R(1.16 * 300.0) / R(1.16)))
+    rd, kappa, grav = ld(R(287.05)), ld(R(0.2854)), ld(R(9.81))
+    zc, idz = grid.metric(1).astype(ld), grid.metric(3).astype(ld)
+
+    def density(p):
+        return p / (rd * th * (p / 1e5) ** kappa)
+
+    p = np.empty((nz, ny, nx), ld)
+    r = np.empty_like(p)
+    p[0] = 1e5 * (rho * rd * th / 1e5) ** (1 / (1 - kappa))
+    r[0] = density(p[0])
+    for k in range(1, nz):
+        dz = zc[k] - zc[k - 1]
+        p[k] = p[k - 1] - grav * r[k - 1] * dz
+        for _ in range(4):
+            p[k] = p[k - 1] - grav * (r[k - 1] + density(p[k])) * dz / 2
+        r[k] = density(p[k])
+    want = ld(R(dt)) * ((p[1:] - p[:-1]) * idz[1:nz] - grav * (2 * rho - r[1:] - r[:-1]) / 2)
+    bound = dt * idz[1:nz] * np.spacing(R(0.99e5)) * ld(0.55)
+    err = np.abs(st.get(O.MOM_W)[1:nz] - want)
+    assert (err <= bound).all(), float((err / bound).max())
