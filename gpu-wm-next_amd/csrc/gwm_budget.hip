@@ -211,6 +211,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
             const double th = CHECK ? ft / d : quot(ft, d, recip(d));
             if (finite2<CHECK>(ft, th)) ath.ext(th);
             else ++ath.bad;
+            if (!CHECK) ath.s += th;  // shows a theta that is not finite
           });
     });
     ar = block_join(ar, sh);
@@ -219,7 +220,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
     put(out, ar);
     put(out + 5, at);
     put(out + 10, ath);
-    return isfinite(ar.s) && isfinite(at.s) && isfinite(ath.mx) && isfinite(ath.mn);
+    return isfinite(ar.s) && isfinite(at.s) && isfinite(ath.s);
   } else if (job <= 3) {
     const R* f = a.face[job - 1];
     const int fx = g.nx + (job == 1), fy = g.ny + (job == 2), fz = g.nz + (job == 3);

@@ -69,3 +69,19 @@ def test_budget_sums_on_ragged_sizes(nx, ny, nz, ntr, prec, form):
     st.set(4, bad)
     s = st.summary()
     assert s["nonfinite_values"] == 2 and np.isnan(s["w_min"]) and np.isfinite(s["u_max"])
+
+
+def test_overflowing_theta_is_reported():
+    """rho theta and rho finite, their quotient not: the field's extremes are
+    NaN, the count of non-finite prognostic values is zero."""
+    ctx = G.Context(0, G.F64)
+    st = G.State(G.Grid(ctx, 66, 5, 3), 1)
+    for f, v in ((0, 1.0), (1, 300.0), (16, 0.01)):
+        st.fill(f, v)
+    rt, rho = st.get(1), st.get(0)
+    rt[2, 4, 65], rho[2, 4, 65] = 1e300, 1e-10
+    st.set(1, rt)
+    st.set(0, rho)
+    s = st.summary()
+    assert np.isnan(s["theta_min"]) and np.isnan(s["theta_max"]) and s["nonfinite_values"] == 0
+    assert s["rho_min"] == 1e-10 and s["qv_max"] == 0.01 / 1e-10
