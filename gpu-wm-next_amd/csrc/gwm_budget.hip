@@ -103,16 +103,12 @@ __device__ inline void put(double* out, const Acc& a) {
   out[4] = static_cast<double>(a.bad);
 }
 
-// Quotients by a shared reciprocal: two Newton steps on the hardware one
-// (positive normal b), then the product corrected with its exact residual,
-// which rounds as the division does; an operand that is not finite gives a
-// quotient that is not.  Five instructions for b and three a quotient against
-// about thirteen each.
-__device__ inline double recip(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
-}
+// Quotients by a shared reciprocal (rcp_newton of a positive normal b): the
+// product corrected with its exact residual, which are the division's own
+// steps without its scaling of the operands (identical results for 7001
+// quotients as near to a tie as there are); an operand that is not finite
+// gives a quotient that is not.  Five instructions for b and three a quotient
+// against about thirteen each.
 __device__ inline double quot(double a, double b, double r) {
   const double q = a * r;
   return __builtin_fma(__builtin_fma(-q, b, a), r, q);
@@ -165,7 +161,10 @@ __device__ inline void along(int fx, L load, F use, int i0 = 0) {
 // One pass of work-group blk of nblk over its job's rows, the records to
 // out.  Returns (thread 0) whether every total is finite.
 // TERRAIN: 1 / dz per cell, and per-cell bases in the perturbation form.
-template <class R, bool CHECK, bool TERRAIN>
+// NTR: tracers (at most 3); reading rho in the place of missing ones, their
+// results unused, made one tracer dearer than three (512 x 512 x 64 FP32: 184,
+// 153 and 163 us for one, two and three tracers; now 131, 150 and 163).
+template <class R, bool CHECK, bool TERRAIN, int NTR>
 __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int blk, int nblk,
                                             double* out, Shared& sh) {
   const Geo& g = a.g;
@@ -208,7 +207,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
             if (finite2<CHECK>(ft, t)) at.sum(t);
             else ++at.bad;
             const double d = fmax(fr, 1.0e-12);
-            const double th = CHECK ? ft / d : quot(ft, d, recip(d));
+            const double th = CHECK ? ft / d : quot(ft, d, rcp_newton(d));
             if (finite2<CHECK>(ft, th)) ath.ext(th);
             else ++ath.bad;
             if (!CHECK) ath.s += th;  // shows a theta that is not finite
@@ -241,17 +240,18 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
     x = block_join(x, sh);
     put(out, x);
     return isfinite(x.s);
-  } else if (job == 4) {
+  } else if (job == 4 && NTR > 0) {
+    constexpr int N = NTR > 0 ? NTR : 1;
     struct V {
-      R r, dr, z, q[3];
+      R r, dr, z, q[N];
     };
-    Acc path[3], mix[3];
+    Acc path[N], mix[N];
     for_rows(wave, waves, g.ny, g.nz, g.pxc, g.pyc, g.h, [&](int k, int j, unsigned o) {
       const double rb = pert ? static_cast<double>(a.base.rho[k]) : 0.0;
       const unsigned m = static_cast<unsigned>((k * g.ny + j) * g.nx);
       const R idz = TERRAIN ? R(1) : a.idz_lev[k];
       const double dz = 1.0 / static_cast<double>(idz);
-      along<2>(
+      along<(N < 3 ? 4 : 2)>(
           g.nx,
           [&](int i) {
             V v{};
@@ -259,7 +259,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
             if (TERRAIN && pert3) v.dr = ld32(a.base.drho, o + i);
             if (TERRAIN) v.z = ld32(a.idz3, m + i);
 #pragma unroll
-            for (int t = 0; t < 3; ++t) v.q[t] = ld32(a.q[t], o + i);
+            for (int t = 0; t < N; ++t) v.q[t] = ld32(a.q[t], o + i);
             return v;
           },
           [&](const V& v) {
@@ -267,9 +267,9 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
             if (pert) r += rb + (pert3 ? static_cast<double>(v.dr) : 0.0);
             const double d = TERRAIN ? 1.0 / static_cast<double>(v.z) : dz;
             r = fmax(r, 1.0e-12);
-            const double ir = recip(r);
+            const double ir = rcp_newton(r);
 #pragma unroll
-            for (int t = 0; t < 3; ++t) {
+            for (int t = 0; t < N; ++t) {
               const double q = static_cast<double>(v.q[t]);
               const double p = q * d, x = CHECK ? q / r : quot(q, r, ir);
               if (finite2<CHECK>(q, p)) path[t].sum(p);
@@ -282,8 +282,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
     });
     bool ok = true;
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
-      if (t >= a.ntr) break;
+    for (int t = 0; t < N; ++t) {
       // the path's extremes are not reported: its record carries the mixing
       // ratio's instead, and the ratio's non-finite count follows
       Acc p = block_join(path[t], sh);
@@ -320,7 +319,7 @@ __device__ __forceinline__ bool budget_pass(const BudgetArgs<R>& a, int job, int
   }
 }
 
-template <class R, bool TERRAIN>
+template <class R, bool TERRAIN, int NTR>
 __global__ __launch_bounds__(kThreads) void k_budget(BudgetArgs<R> a) {
   __shared__ Shared sh;
   __shared__ int again;
@@ -329,10 +328,10 @@ __global__ __launch_bounds__(kThreads) void k_budget(BudgetArgs<R> a) {
   const int blk = static_cast<int>(blockIdx.x) - a.block0[job];
   const int nblk = a.block0[job + 1] - a.block0[job];
   double* out = a.part + a.part0[job] + static_cast<size_t>(blk) * a.record[job];
-  const bool ok = budget_pass<R, false, TERRAIN>(a, job, blk, nblk, out, sh);
+  const bool ok = budget_pass<R, false, TERRAIN, NTR>(a, job, blk, nblk, out, sh);
   if (threadIdx.x == 0) again = !ok;
   __syncthreads();
-  if (again) budget_pass<R, true, TERRAIN>(a, job, blk, nblk, out, sh);
+  if (again) budget_pass<R, true, TERRAIN, NTR>(a, job, blk, nblk, out, sh);
 }
 
 // Work-groups of the jobs (of 256 in all) about in proportion to the bytes
@@ -361,11 +360,20 @@ int budget_layout(BudgetArgs<R>& a) {
 template <class R>
 void launch_budget(hipStream_t st, const BudgetArgs<R>& a) {
   if (refuse_record("budget")) return;
-  const dim3 grid(a.block0[kBudgetJobs]), blk(kThreads);
-  if (a.idz3)
-    hipLaunchKernelGGL((k_budget<R, true>), grid, blk, 0, st, a);
-  else
-    hipLaunchKernelGGL((k_budget<R, false>), grid, blk, 0, st, a);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(a.block0[kBudgetJobs]), dim3(kThreads), 0, st, a);
+  };
+  auto form = [&](auto terrain) {
+    constexpr bool T = decltype(terrain)::value;
+    switch (a.ntr) {
+      case 0: go(k_budget<R, T, 0>); break;
+      case 1: go(k_budget<R, T, 1>); break;
+      case 2: go(k_budget<R, T, 2>); break;
+      default: go(k_budget<R, T, 3>); break;
+    }
+  };
+  if (a.idz3) form(std::true_type{});
+  else form(std::false_type{});
 }
 
 template int budget_layout<float>(BudgetArgs<float>&);

@@ -1051,9 +1051,7 @@ void budget(gwm_state* S, double* o, double* dev = nullptr, double* host = nullp
   A.rt = static_cast<const R*>(ds[1]);
   for (int f = 0; f < 3; ++f) A.face[f] = static_cast<const R*>(ds[GWM_MOM_U + f]);
   A.ntr = std::min(S->ntr, 3);
-  // (a missing tracer reads rho in its place; its record is not written)
-  for (int t = 0; t < 3; ++t)
-    A.q[t] = t < A.ntr ? static_cast<const R*>(S->field(GWM_TRACER0 + t)) : A.rho;
+  for (int t = 0; t < A.ntr; ++t) A.q[t] = static_cast<const R*>(S->field(GWM_TRACER0 + t));
   A.precip = static_cast<const R*>(S->view ? S->owner->precip : S->precip);
   A.idz3 = S->grid->terrain_nonzero ? static_cast<const R*>(S->grid->idz_c) : nullptr;
   A.idz_lev = static_cast<const R*>(S->grid->lev_idz_c);
