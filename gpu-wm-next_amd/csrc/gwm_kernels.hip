@@ -260,7 +260,8 @@ __global__ void k_rebuild_rt(Geo g, const R* rho, const R* th, R* rt, Base<R> ba
 // post-microphysics rain exactly like the reference's qr_old copy.
 //
 // A wave is 64 columns, and the waves of a work-group share them, each with a
-// chunk of the levels (blockDim.y chunks): what falls into a chunk depends on
+// chunk of the levels (blockDim.y chunks; blockDim.z rows of such waves: one,
+// but in the widest batched members): what falls into a chunk depends on
 // the level above it only, which the wave adjusts a second time for itself.
 // The update is in place, so every wave reads that level before any writes
 // (they are all in the work-group).  One thread per column left too few waves
@@ -271,9 +272,10 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
   const Geo g = a.g;
   int bx, by;
   xcd_block2d(vb, bx, by);
-  const int ic = bx * 64 + static_cast<int>(threadIdx.x), j = by;
-  const bool in = ic < g.nx;
-  const int i = in ? ic : g.nx - 1;
+  const int ic = bx * 64 + static_cast<int>(threadIdx.x);
+  const int jc = by * static_cast<int>(blockDim.z) + static_cast<int>(threadIdx.z);
+  const bool in = ic < g.nx && jc < g.ny;
+  const int i = ic < g.nx ? ic : g.nx - 1, j = jc < g.ny ? jc : g.ny - 1;
   const int nch = static_cast<int>(blockDim.y), chunk = static_cast<int>(threadIdx.y);
   const int k0 = (g.nz * chunk) / nch, k1 = (g.nz * (chunk + 1)) / nch;
   const R dt = a.dt;
@@ -710,15 +712,16 @@ void launch_warm_rain(hipStream_t st, const WarmRainArgs<R>& a, bool terrain) {
   const long waves = static_cast<long>(gr.x) * gr.y;
   int chunks = waves >= 2048 ? 2 : waves >= 128 ? 4 : 8;
   while (chunks > 1 && a.g.nz < 4 * chunks) chunks /= 2;
-  const dim3 b(64, chunks, 1);
   if (recorder()) {
     const void* fn = terrain ? reinterpret_cast<const void*>(&k_warm_rain_batch<R, true>)
                              : reinterpret_cast<const void*>(&k_warm_rain_batch<R, false>);
-    record_launch(fn, b, 0, WarmRainItem<R>{a, 0, 0}, static_cast<int>(gr.x),
-                  static_cast<int>(gr.y));
+    // (a batched launch numbers a member's work-groups in kBatchBlockBits bits)
+    const bool wide = waves >= (1L << kBatchBlockBits);
+    record_launch(fn, dim3(64, chunks, wide ? 4 : 1), 0, WarmRainItem<R>{a, 0, 0},
+                  static_cast<int>(gr.x), static_cast<int>(wide ? (gr.y + 3) / 4 : gr.y));
     return;
   }
-  const dim3 flat(gr.x * gr.y);
+  const dim3 b(64, chunks, 1), flat(gr.x * gr.y);
   if (terrain)
     hipLaunchKernelGGL((k_warm_rain<R, true>), flat, b, 0, st, a);
   else

@@ -46,3 +46,29 @@ def test_chunk_counts_agree(nz, prec, metric):
     for k in first:
         want = w.get(k)
         assert np.abs(first[k] - want).max() <= 4 * tol * max(np.abs(want).max(), 1e-6), k
+
+
+def test_ensemble_member_of_a_million_rows():
+    """A batched launch numbers a member's work-groups in 20 bits: a member
+    whose warm rain has 2^20 + 1 rows of waves batches beside a small one
+    (rows in fours, the last one short), and both equal steps by themselves."""
+    ctx = G.Context(0, G.F32)
+    cfg, wr = G.step_config(0.5, 2), G.warm_rain_config(dt=0.5, rain_terminal_velocity=5.0)
+    members, alone = [], []
+    for e, (nx, ny, nz) in enumerate(((2, 2 ** 20 + 1, 1), (40, 24, 9))):
+        grid = G.Grid(ctx, nx, ny, nz, z_interfaces=np.linspace(0.0, 500.0 * nz, nz + 1))
+        for group in (members, alone):
+            rng = np.random.default_rng(e)
+            st = G.State(grid, 3)
+            st.init_constant_n(u=3.0)
+            rho = st.get(O.RHO)
+            for t, q in enumerate((2e-2, 2e-3, 2e-3)):
+                st.set(O.TRACER0 + t, rho * (q * rng.random(rho.shape)).astype(ctx.dtype))
+            group.append(st)
+    G.ensemble_steps(members, cfg, wr, 3)
+    for m, a in zip(members, alone):
+        for _ in range(3):
+            a.moist_step(cfg, wr)
+        for k in (0, 1, 2, 3, 4, 16, 17, 18, G.PRECIP):
+            np.testing.assert_array_equal(m.get(k), a.get(k), err_msg=str(k))
+        assert a.get(G.PRECIP).max() > 0
