@@ -264,10 +264,12 @@ __global__ void k_rebuild_rt(Geo g, const R* rho, const R* th, R* rt, Base<R> ba
 // but in the widest batched members): what falls into a chunk depends on
 // the level above it only, which the wave adjusts a second time for itself.
 // The update is in place, so every wave reads that level before any writes
-// (they are all in the work-group).  One thread per column left too few waves
-// to cover the loads (figures at the launcher's rule).
+// (they are all in the work-group).  One thread per column leaves too few
+// waves to cover the loads of small and deep grids (figures at the launcher's
+// rule).  CHUNKED: more chunks than one; whole columns take a kernel of their
+// own, which the second adjustment's code made 3 to 5 % slower.
 // ===========================================================================
-template <class R, bool TERRAIN>
+template <class R, bool TERRAIN, bool CHUNKED>
 __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const VBlock& vb) {
   const Geo g = a.g;
   int bx, by;
@@ -276,7 +278,8 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
   const int jc = by * static_cast<int>(blockDim.z) + static_cast<int>(threadIdx.z);
   const bool in = ic < g.nx && jc < g.ny;
   const int i = ic < g.nx ? ic : g.nx - 1, j = jc < g.ny ? jc : g.ny - 1;
-  const int nch = static_cast<int>(blockDim.y), chunk = static_cast<int>(threadIdx.y);
+  const int nch = CHUNKED ? static_cast<int>(blockDim.y) : 1;
+  const int chunk = CHUNKED ? static_cast<int>(threadIdx.y) : 0;
   const int k0 = (g.nz * chunk) / nch, k1 = (g.nz * (chunk + 1)) / nch;
   const R dt = a.dt;
   R inc = 0;
@@ -329,16 +332,16 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
   // arithmetic.
   size_t c = g.cell(i, j, k1 - 1);
   Lv l1{}, l2{}, l3{}, above{};
-  if (k1 < g.nz) above = load(c + plane);
+  if (CHUNKED && k1 < g.nz) above = load(c + plane);
   if (k1 > k0) l1 = load(c);
   if (k1 - 1 > k0) l2 = load(c - plane);
   if (k1 - 2 > k0) l3 = load(c - 2 * plane);
-  if (nch > 1) {
+  if constexpr (CHUNKED) {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the level above has been read
     __syncthreads();
   }
   if (!in) return;
-  if (k1 < g.nz && (nominal || metric)) fall(adjust(above, k1).rqr, k1);
+  if (CHUNKED && k1 < g.nz && (nominal || metric)) fall(adjust(above, k1).rqr, k1);
   for (int k = k1 - 1; k >= k0; --k) {
     const Lv cur = l1;
     l1 = l2;
@@ -355,20 +358,21 @@ __device__ __forceinline__ void warm_rain_body(const WarmRainArgs<R>& a, const V
   if (nominal || metric) a.precip[static_cast<size_t>(j) * g.nx + i] += inc;
 }
 
-template <class R, bool TERRAIN>
+template <class R, bool TERRAIN, bool CHUNKED>
 __global__ __launch_bounds__(512) void k_warm_rain(WarmRainArgs<R> a) {
   // (a row of 64-column waves after the other in x: the launch's y extent
   // would limit the rows)
   const int gx = (a.g.nx + 63) / 64, b = static_cast<int>(blockIdx.x);
-  warm_rain_body<R, TERRAIN>(a, VBlock{b % gx, b / gx, gx, a.g.ny});
+  const int rows = static_cast<int>(blockDim.z);
+  warm_rain_body<R, TERRAIN, CHUNKED>(a, VBlock{b % gx, b / gx, gx, (a.g.ny + rows - 1) / rows});
 }
-template <class R, bool TERRAIN>
+template <class R, bool TERRAIN, bool CHUNKED>
 __global__ __launch_bounds__(512) void k_warm_rain_batch(const WarmRainItem<R>* items, BatchMap bm) {
   VBlock vb;
   const WarmRainItem<R>* it = batch_member(items, bm, vb);
   if (!it) return;
   const WarmRainArgs<R> a = it->a;
-  warm_rain_body<R, TERRAIN>(a, vb);
+  warm_rain_body<R, TERRAIN, CHUNKED>(a, vb);
 }
 
 // ===========================================================================
@@ -703,29 +707,41 @@ void launch_rebuild_rt(hipStream_t st, const Geo& g, const R* rho, const R* th, 
 }
 template <class R>
 void launch_warm_rain(hipStream_t st, const WarmRainArgs<R>& a, bool terrain) {
-  // Enough waves to cover the loads, and no more than that (each chunk costs a
-  // second adjustment of a level): by the number of 64-column waves.  Measured
-  // with 1 / 2 / 4 / 8 chunks (us): 4096 waves of 64 levels in FP32 193, 150,
-  // 158, 177; 1024 in FP64 237, 163, 125, 121; eight members of 192 to 896
-  // waves in one launch 152, 124, 119, 126; 64 waves of 40 levels 38, 22, 13, 10.
+  // Enough waves to cover the loads, and no more than that: each chunk costs a
+  // second adjustment of a level, so chunks keep some levels too.  By the
+  // number of 64-column waves (of a batched launch, the member's).  Measured
+  // with 1 / 2 / 4 / 8 chunks (us, nominal fallout):
+  //   waves x levels   FP32                     FP64
+  //   64 x 40          34, 21, 13, 11           46, 28, 17, 17
+  //   1024 x 16        20, 16, 16, 17           26.6, 26.1, 28.5, 36
+  //   1024 x 64        59, 44, 40, 41           86, 78, 78, 88
+  //   4096 x 8         22, 24, 28, 28           42, 49, 60, 59
+  //   4096 x 24        54, 56                   112, 113
+  //   4096 x 64        144, 138, 146, 155       294, 297, 317, 342
+  //   16384 x 8        65, 76, 91, 91           154, 183, 217, 219
+  //   16384 x 32       285, 285, 284, 307       558, 586, 623, 759
+  constexpr bool f64 = sizeof(R) == 8;
   const dim3 gr((a.g.nx + 63) / 64, a.g.ny);
   const long waves = static_cast<long>(gr.x) * gr.y;
-  int chunks = waves >= 2048 ? 2 : waves >= 128 ? 4 : 8;
-  while (chunks > 1 && a.g.nz < 4 * chunks) chunks /= 2;
-  if (recorder()) {
-    const void* fn = terrain ? reinterpret_cast<const void*>(&k_warm_rain_batch<R, true>)
-                             : reinterpret_cast<const void*>(&k_warm_rain_batch<R, false>);
-    // (a batched launch numbers a member's work-groups in kBatchBlockBits bits)
-    const bool wide = waves >= (1L << kBatchBlockBits);
-    record_launch(fn, dim3(64, chunks, wide ? 4 : 1), 0, WarmRainItem<R>{a, 0, 0},
-                  static_cast<int>(gr.x), static_cast<int>(wide ? (gr.y + 3) / 4 : gr.y));
-    return;
-  }
-  const dim3 b(64, chunks, 1), flat(gr.x * gr.y);
-  if (terrain)
-    hipLaunchKernelGGL((k_warm_rain<R, true>), flat, b, 0, st, a);
-  else
-    hipLaunchKernelGGL((k_warm_rain<R, false>), flat, b, 0, st, a);
+  int chunks = waves >= 2048 ? (f64 ? 1 : 2) : waves >= 128 ? 4 : 8;
+  const int levels = waves >= 2048 ? 16 : f64 && waves >= 128 ? 8 : 4;  // of a chunk
+  while (chunks > 1 && a.g.nz < levels * chunks) chunks /= 2;
+  // (a batched launch numbers a member's work-groups in kBatchBlockBits bits)
+  const int rows = recorder() && waves >= (1L << kBatchBlockBits) ? 4 : 1;
+  const dim3 b(64, chunks, rows);
+  const unsigned gy = (gr.y + rows - 1) / rows;
+  auto go = [&](auto t, auto c) {
+    constexpr bool T = decltype(t)::value, C = decltype(c)::value;
+    if (recorder())
+      record_launch(reinterpret_cast<const void*>(&k_warm_rain_batch<R, T, C>), b, 0,
+                    WarmRainItem<R>{a, 0, 0}, static_cast<int>(gr.x), static_cast<int>(gy));
+    else
+      hipLaunchKernelGGL((k_warm_rain<R, T, C>), dim3(gr.x * gy), b, 0, st, a);
+  };
+  using std::false_type;
+  using std::true_type;
+  if (terrain) chunks > 1 ? go(true_type{}, true_type{}) : go(true_type{}, false_type{});
+  else chunks > 1 ? go(false_type{}, true_type{}) : go(false_type{}, false_type{});
 }
 template <class R>
 void launch_halo_fill(hipStream_t st, const Geo& g, int orient, R* f) {

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nz,prec,metric", [(1, G.F64, True), (7, G.F32, True), (9, G.F64, False),
-                                            (17, G.F32, False), (33, G.F64, True)])
+                                            (17, G.F32, False), (33, G.F64, True),
+                                            (33, G.F32, False)])
 def test_chunk_counts_agree(nz, prec, metric):
     nx, ny = 70, 4
     ctx = G.Context(0, prec)
