@@ -971,8 +971,11 @@ void launch_fast_kind(hipStream_t st, const FastArgs<R>& a, int nkc, double* par
   const int tx = (a.g.nx + TX - 1) / TX, ty = (a.g.ny + TYV - 1) / TYV;
   const int tiles = tx * ty;
   const dim3 grid(tiles * nkc), blk(TX, TYV, 1);
-  // per-level LDS: the longest chunk plus the levels below and above it
-  const size_t lds = static_cast<size_t>((a.g.nz + nkc - 1) / nkc + 3) * NLV * sizeof(R);
+  // per-level LDS: the longest chunk plus the levels below and above it (the
+  // column reference form has no per-level values)
+  const size_t lds = FORM == 4 + REF_COLUMN
+                         ? 0
+                         : static_cast<size_t>((a.g.nz + nkc - 1) / nkc + 3) * NLV * sizeof(R);
   const int kind = (a.first ? 1 : 0) | (a.last ? 2 : 0);
   if (recorder()) {
     const void* fns[4] = {reinterpret_cast<const void*>(&k_fast_column_batch<R, FORM, 0, TYV>),
