@@ -565,7 +565,7 @@ void level_theta_ref(gwm_state* S, const R* rho, const R* rt, gwm::SlowArgs<R>& 
 // back-to-back pairs while timing slower launch by launch.
 template <class Launch>
 int pick_chunks(gwm_ctx* ctx, const char* kname, const Geo& g, int variant, Launch&& launch,
-                int shapes = 1, bool whole_columns = false, bool fine = false) {
+                int shapes = 1, bool fine = false) {
   if (ctx->force_chunks > 0) return ctx->force_chunks;
   char key[160];
   std::snprintf(key, sizeof key, "%s:%dx%dx%d:%s:%d", kname, g.nx, g.ny, g.nz,
@@ -581,7 +581,7 @@ int pick_chunks(gwm_ctx* ctx, const char* kname, const Geo& g, int variant, Laun
   std::vector<int> cands;
   for (int sh = 0; sh < shapes; ++sh)
     for (int n : {1, 2, 3, 4, 6, 8, 12})
-      if (n == 1 || (!whole_columns && g.nz / n >= 4 && (fine || (n & (n - 1)) == 0)))
+      if (n == 1 || (g.nz / n >= 4 && (fine || (n & (n - 1)) == 0)))
         cands.push_back(n | (sh << 4));
   std::vector<float> t_min(cands.size(), 1e30f);
   for (int round = 0; round < 3; ++round)
@@ -745,7 +745,7 @@ void slow_stage(gwm_state* S, const gwm_step_config& c, void* const* in, void* c
   };
   const int nkc = pick_chunks(S->ctx, "slow_column", g,
                               (S->grid->terrain_nonzero ? 1 : 0) + 2 * mode + (S->pert3 ? 16 : 0),
-                              run, 1, false, true);
+                              run, 1, true);
   Timed t(S->ctx, "slow_stage");
   run(nkc);
 }
@@ -992,8 +992,7 @@ void tracers_ssprk3(gwm_state* S, const gwm_step_config& c, int bmode,
       gwm::launch_tracer_column<R>(S->ctx->stream, a, S->grid->terrain_nonzero, n);
     };
     const int nkc = pick_chunks(S->ctx, "tracer_column", g,
-                                (S->grid->terrain_nonzero ? 1 : 0) + 2 * S->ntr, run, 1, false,
-                                true);
+                                (S->grid->terrain_nonzero ? 1 : 0) + 2 * S->ntr, run, 1, true);
     Timed tt(S->ctx, "tracer_stage");
     run(nkc);
   };
