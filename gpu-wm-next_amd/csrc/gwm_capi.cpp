@@ -472,15 +472,16 @@ struct gwm_state {
     return sur_queue;
   }
   // Partial-sum buffer of the step's level means (both uses fit).
-  // Two halves: a substep that sums its own level partials reads one while it
-  // writes the next substep's to the other.
+  // Where kernels sum level partials themselves (inline_parts, by either
+  // count), two halves: a substep reads one while it writes the next one's to
+  // the other.  Elsewhere a launch has summed them before they are overwritten.
   double* level_part(int half) {
     const Geo& gg = g();
-    const size_t per = std::max<size_t>(gwm::fast_column_parts(gg.nx, gg.ny),
-                                        gwm::level_partials_chunks(gg.ny));
-    const size_t n = static_cast<size_t>(gg.nz) * per * 2;
-    if (!step_part) step_part = static_cast<double*>(dalloc(2 * n * sizeof(double)));
-    return step_part + (half & 1 ? n : 0);
+    const int few = gwm::level_partials_chunks(gg.ny), many = gwm::fast_column_parts(gg.nx, gg.ny);
+    const bool two = gwm::inline_size(gg, std::min(few, many));
+    const size_t n = static_cast<size_t>(gg.nz) * std::max(few, many) * 2;
+    if (!step_part) step_part = static_cast<double*>(dalloc((two ? 2 : 1) * n * sizeof(double)));
+    return step_part + (two && (half & 1) ? n : 0);
   }
 };
 
@@ -520,8 +521,7 @@ void ensure_synced(gwm_state* S, void** fs) {
 // Level means of small grids are left to the kernels that use them; not in a
 // recorded (batched) step, whose members must launch the same sequence.
 bool inline_parts(const Geo& g, int nparts) {
-  return nparts <= gwm::kInlineParts &&
-         static_cast<long>(g.nx) * g.ny * g.nz <= gwm::kInlineCells && !gwm::recorder();
+  return gwm::inline_size(g, nparts) && !gwm::recorder();
 }
 
 template <class R>

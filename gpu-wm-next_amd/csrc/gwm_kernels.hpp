@@ -125,6 +125,9 @@ void launch_level_partials(hipStream_t st, const Geo& g, const R* rho, const R* 
 // pass, lost 5 % with it.
 constexpr int kInlineParts = 128;
 constexpr long kInlineCells = 1L << 20;
+inline bool inline_size(const Geo& g, int nparts) {
+  return nparts <= kInlineParts && static_cast<long>(g.nx) * g.ny * g.nz <= kInlineCells;
+}
 // Partials per level written by launch_level_partials for ny rows.
 int level_partials_chunks(int ny);
 template <class R>
