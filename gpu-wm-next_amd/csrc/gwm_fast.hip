@@ -14,13 +14,13 @@
 // cell and level into an LDS ring of four planes (levels k-1 .. k+2); the
 // plane two levels ahead and the face momenta one level ahead are loaded into
 // registers an iteration early, so their global loads overlap the current
-// level's arithmetic.  The w face above the cell and the column reference are
-// carried in registers, so each face is computed once.  One barrier per
-// level.  Splitting the column into chunks (chosen by the autotuner) gives
-// the chip more independent work-groups; a chunk recomputes its bottom w face
-// from the level below.  Terrain has a march of its own below, with the column
-// hydrostatic reference (a recurrence from the ground) in a kernel before it.
-// Work-group b is remapped so that each XCD (which receives every eighth work-group) owns a
+// level's arithmetic.  The w face above the cell is carried in registers, so
+// each face is computed once.  One barrier per level.  Splitting the column
+// into chunks (chosen by the autotuner) gives the chip more independent
+// work-groups; a chunk recomputes its bottom w face from the level below.
+// Terrain has a march of its own below, with the column hydrostatic reference
+// (a recurrence from the ground) in a kernel before it.  Work-group b is
+// remapped so that each XCD (which receives every eighth work-group) owns a
 // contiguous band of tiles and the ring rows shared by neighbouring tiles hit
 // the same L2.
 //
@@ -758,7 +758,7 @@ __device__ __forceinline__ void fast_terrain_body(const FastArgs<R>& a, int tile
 //
 // The chain of dependent operations is what bounds it: five powers and ten
 // quotients a level, carried in the substep's own whole-column march, made an
-// FP64 substep of 151 x 97 x 40 take 257 us; this kernel takes 20 of the 48
+// FP64 substep of 151 x 97 x 40 take 257 us; this kernel takes 18 of the 47
 // it takes now.  Here each density is a series about the cell's own state,
 // which needs no power: with p_a = EOS(rho_a, theta), rho(p, theta) = rho_a
 // (p / p_a)^(1 - kappa), and u = p / p_a - 1 is small as the reference

@@ -379,11 +379,9 @@ int gwm_plan_view(gwm_state* state, int slice_k, int steps, double dt, int with_
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  The reduction partials live
  * in a static device array of 4096 doubles (32 KiB per GPU, held until the
- * process ends; the budget needs fewer of them for any grid size), host
- * staging is on the stack, and the precipitation bucket is reduced on the
- * device.  Same slots as gwm_budget_sums: counts, extremes and the
- * non-finite count agree exactly, sums to rounding (the bucket is summed in
- * another order).  Calls that overlap on one GPU share the array and race;
+ * process ends; the budget needs fewer of them for any grid size) and host
+ * staging is on the stack.  Same launch, slots and results as
+ * gwm_budget_sums.  Calls that overlap on one GPU share the array and race;
  * each call synchronises the state's stream before it returns. */
 int gwm_budget_sums_noalloc(gwm_state* state, double* out);
 

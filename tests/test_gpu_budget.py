@@ -1,7 +1,8 @@
 """The one-launch budget sums against numpy on ragged sizes: rows shorter and
 longer than a wave, a last batch of loads that ends inside it, fewer rows than
 waves, every tracer count, terrain and the perturbation form.  Extremes and
-counts are exact (single IEEE operations on the same values); sums are
+counts are exact (single operations on the same values; the device's FP64
+division misses numpy's only beside a tie, closer than 2^-52 ulp); sums are
 compensated on both sides, so they agree to the rounding of the result and of
 each term (2^-53 of the sum of magnitudes bounds both)."""
 import math

@@ -579,10 +579,11 @@ def test_downward_march_does_not_change_results(ctx32, perturbation, ty4):
 
 @pytest.mark.parametrize("prec", [8, 4])
 def test_column_reference_tile_heights_do_not_change_results(ctx32, ctx64, prec):
-    """On terrain the fast kernel keeps whole columns (the column reference
-    is a recurrence from the ground) and its tile height (8 or 4 rows) is
-    autotuned; both give bit-identical states on an open-x ridge grid whose
-    8-row tiles end in a partial one."""
+    """On terrain the fast kernel's tile height (8 or 4 rows) is autotuned
+    like its level chunks (the column reference, a recurrence from the ground,
+    has a kernel of its own); both heights give bit-identical states on an
+    open-x ridge grid whose 8-row tiles end in a partial one, here in whole
+    columns."""
     ctx = ctx_for(prec, ctx32, ctx64)
     nx, ny, nz, dx = 96, 20, 16, 2000.0
     zi = G.stretched_levels(nz, 50.0, 600.0, 8000.0)
